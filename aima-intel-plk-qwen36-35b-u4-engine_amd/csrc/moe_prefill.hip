@@ -5,15 +5,16 @@
 //    assignment index, the order of the reference's host BuildGroupedSchedule
 //    (grouped_s8_u4_prefill_runtime.cpp:231-346), so the schedule is
 //    deterministic and bit-comparable with the CPU restatement.  The scan
-//    also emits the M tiles (up to 256 rows of one expert; the shared expert
-//    covers all T tokens), ordered by height, tallest first.
+//    also emits the M tiles (up to 256 rows of one expert, or 16 in small calls;
+//    the shared expert covers all T tokens), ordered by height, tallest first.
 // 2. Grouped gate/up GEMM (MFMA v_mfma_f32_32x32x16_f16): per tile, the token
 //    rows are gathered into LDS; each wave dequantizes its own 32 weight rows
 //    straight into MFMA operands as f16 (q - z) * s and multiplies them with
-//    every token row of the tile.  The SwiGLU epilogue scales each row by its
-//    router weight (1 for the shared expert) and writes f16 [rows][I].
-// 3. Grouped down GEMM, same structure over K = I; its output rows are then
-//    the weighted contributions, written as f16 [rows][H].
+//    every token row of the tile; tiles of at most 32 rows multiply the integer
+//    codes instead (grouped_thin.h).  The SwiGLU epilogue writes f16 [rows][I].
+// 3. Grouped down GEMM, same structure over K = I; its output rows times their
+//    router weights (1 for the shared expert) are the contributions, written as
+//    f16 [rows][H].
 // 4. Combine: per token, the k contributions in rank order, plus the
 //    sigmoid-gated shared row, plus the residual, summed in f32 and rounded
 //    to f16.
@@ -25,6 +26,7 @@
 // grouped_s8_u4_f16_contribution_moe.cl:831-845); MI355X runs dense f16 and
 // bf16 MFMA at the same rate.
 #include "common.h"
+#include "grouped_thin.h"
 
 #include <math.h>
 
@@ -33,9 +35,10 @@
 namespace aima {
 
 constexpr int kBM = 256;            // rows per M tile (8 MFMA blocks of 32)
+constexpr int kMinTileLog2 = 4;     // rows of the thinnest tiles
 constexpr int kSchedBlock = 1024;   // assignments per schedule block
 constexpr int kMaxExperts = 1024;
-constexpr int kTileClasses = 8;     // tile heights 32, 64, ..., 256 rows
+constexpr int kTileClasses = 8;     // tile heights in eighths of the tallest
 
 struct PrefillWs {
   uint32_t* err;
@@ -57,7 +60,24 @@ struct PrefillWs {
 struct PrefillDims {
   int64_t T, A, nb, max_tiles;
   int E, k, H, I;
+  int bm_log2;  // rows per M tile: 2^bm_log2
 };
+
+// Most M tiles of `bm` rows: every expert with rows adds at most one partial
+// tile.
+static int64_t tile_bound(const PrefillDims& d, int64_t bm) {
+  return (d.A + bm - 1) / bm + std::min<int64_t>(d.E, d.A) + (d.T + bm - 1) / bm;
+}
+
+// Tile height.  Up to 10 assignments per expert on average, most tiles are
+// thin whatever the height, and 16-row tiles in small blocks (several per CU:
+// grouped_thin_kernel) beat the 512-thread blocks of grouped_gemm_kernel:
+// T = 96 (3 per expert, hidden 2048, inter 512, 256 experts, k = 8) 108
+// against 134 us per call, T = 200 (6.3) 119 against 150, uniform routing.
+// Beyond, an expert's weights are read once per 16 rows for nothing: at 12.5
+// per expert 141 against 160 us if the routing is uniform, but 116 against
+// 109 if it is skewed, 14 per expert 124 against 110.
+static int tile_rows_log2(const PrefillDims& d) { return d.A <= 10 * (int64_t)d.E ? 4 : 8; }
 
 static PrefillDims prefill_dims(const aima_moe_layer* L, int64_t T, int k) {
   PrefillDims d;
@@ -68,8 +88,8 @@ static PrefillDims prefill_dims(const aima_moe_layer* L, int64_t T, int k) {
   d.H = L->hidden;
   d.I = L->inter;
   d.nb = (d.A + kSchedBlock - 1) / kSchedBlock;
-  // every expert with rows adds at most one partial tile
-  d.max_tiles = (d.A + kBM - 1) / kBM + std::min<int64_t>(d.E, d.A) + (T + kBM - 1) / kBM;
+  d.bm_log2 = tile_rows_log2(d);
+  d.max_tiles = tile_bound(d, 1 << d.bm_log2);
   return d;
 }
 
@@ -90,7 +110,9 @@ static size_t prefill_ws_layout(const PrefillDims& d, WsMode mode, void* base, P
   l.tile_count = reinterpret_cast<int32_t*>(hdr ? hdr + 64 : nullptr);
   l.block_base = reinterpret_cast<int32_t*>(take((size_t)d.nb * d.E * 4));
   l.offsets = reinterpret_cast<int32_t*>(take((size_t)d.E * 4));
-  l.tiles = reinterpret_cast<int32_t*>(take((size_t)d.max_tiles * 16));
+  // room for the thinnest tiles, whatever height this call takes: the size
+  // then only grows with the tokens
+  l.tiles = reinterpret_cast<int32_t*>(take((size_t)tile_bound(d, 1 << kMinTileLog2) * 16));
   l.token_map = reinterpret_cast<int32_t*>(take((size_t)d.A * 4));
   l.inverse_map = reinterpret_cast<int32_t*>(take((size_t)d.A * 4));
   l.row_weight = reinterpret_cast<float*>(take((size_t)d.A * 4));
@@ -231,13 +253,15 @@ __device__ void block_exclusive_scan_1024(int (&v)[N], int (&tot)[N], int* smem)
   __syncthreads();
 }
 
-// Tiles of one expert with `total` rows in class c (1..8 MFMA blocks of 32
-// rows): full 256-row tiles are class 8, the remainder tile is class
-// ceil(rem / 32).
-__device__ __forceinline__ int tiles_in_class(int total, int c) {
-  const int rem = total % kBM;
-  const int cls = (rem + 31) / 32;
-  return (c == kTileClasses ? total / kBM : 0) + (cls == c ? 1 : 0);
+// Height class of a remainder tile of `rem` rows (1..8 eighths of the full
+// height; 0 without rows).
+__device__ __forceinline__ int tile_class(int rem, int bm_log2) {
+  return (rem * kTileClasses + (1 << bm_log2) - 1) >> bm_log2;
+}
+// Tiles of one expert with `total` rows in class c: full tiles are class 8.
+__device__ __forceinline__ int tiles_in_class(int total, int c, int bm_log2) {
+  const int rem = total & ((1 << bm_log2) - 1);
+  return (c == kTileClasses ? total >> bm_log2 : 0) + (tile_class(rem, bm_log2) == c ? 1 : 0);
 }
 
 // One block of 1024 threads: thread (p, e) with e = tid % Ep (Ep = E rounded
@@ -246,7 +270,7 @@ __device__ __forceinline__ int tiles_in_class(int total, int c) {
 // into row offsets and into tile positions per class (class 8 first).
 __global__ __launch_bounds__(1024) void sched_scan_kernel(int32_t* __restrict__ block_base,
                                                           int32_t nb, int E, int Ep, int32_t T,
-                                                          int32_t A, int with_shared,
+                                                          int32_t A, int with_shared, int bm_log2,
                                                           int32_t* __restrict__ offsets,
                                                           int32_t* __restrict__ tiles,
                                                           int32_t* __restrict__ tile_count) {
@@ -280,7 +304,7 @@ __global__ __launch_bounds__(1024) void sched_scan_kernel(int32_t* __restrict__ 
   int v[1 + kTileClasses], tot[1 + kTileClasses];
   v[0] = rep ? total : 0;
 #pragma unroll
-  for (int c = 1; c <= kTileClasses; ++c) v[c] = rep ? tiles_in_class(total, c) : 0;
+  for (int c = 1; c <= kTileClasses; ++c) v[c] = rep ? tiles_in_class(total, c, bm_log2) : 0;
   block_exclusive_scan_1024<1 + kTileClasses>(v, tot, smem);
   const int begin = v[0];
   if (rep) offsets[e] = begin + total;
@@ -302,34 +326,35 @@ __global__ __launch_bounds__(1024) void sched_scan_kernel(int32_t* __restrict__ 
   }
   // Tiles, by class (tallest first); the shared expert's tiles follow the
   // routed ones of each class.  An expert has full tiles (class 8) and at
-  // most one remainder tile of class ceil(rem / 32).
+  // most one remainder tile.
   int cbase[kTileClasses + 1];
   int all_tiles = 0;
 #pragma unroll
   for (int c = kTileClasses; c >= 1; --c) {
     cbase[c] = all_tiles;
-    all_tiles += tot[c] + (with_shared ? tiles_in_class(T, c) : 0);
+    all_tiles += tot[c] + (with_shared ? tiles_in_class(T, c, bm_log2) : 0);
   }
   auto place = [&](int ex, int row_begin, int rows_total, int first8, int rem_pos_if_not8) {
-    const int full = rows_total / kBM, rem = rows_total % kBM;
+    const int bm = 1 << bm_log2, full = rows_total >> bm_log2, rem = rows_total & (bm - 1);
     for (int i = 0; i < full; ++i) {
       int32_t* td = tiles + 4 * (int64_t)(first8 + i);
       td[0] = ex;
-      td[1] = row_begin + i * kBM;
-      td[2] = kBM;
+      td[1] = row_begin + i * bm;
+      td[2] = bm;
       td[3] = 0;
     }
     if (rem) {
-      const int at = (rem + 31) / 32 == kTileClasses ? first8 + full : rem_pos_if_not8;
+      const int at =
+          tile_class(rem, bm_log2) == kTileClasses ? first8 + full : rem_pos_if_not8;
       int32_t* td = tiles + 4 * (int64_t)at;
       td[0] = ex;
-      td[1] = row_begin + full * kBM;
+      td[1] = row_begin + full * bm;
       td[2] = rem;
       td[3] = 0;
     }
   };
   auto rem_slot = [&](int rows_total, const int (&prefix)[1 + kTileClasses]) {
-    const int cls = (rows_total % kBM + 31) / 32;
+    const int cls = tile_class(rows_total & ((1 << bm_log2) - 1), bm_log2);
     int pos = 0;
 #pragma unroll
     for (int c = 1; c < kTileClasses; ++c) {
@@ -417,7 +442,7 @@ __device__ __forceinline__ void plain_barrier() {
 // bytes, gathered through the token map) reach LDS by direct global->LDS
 // loads into a two-buffer ring; 16-byte piece p of row r sits in slot
 // p ^ (r & 15), which keeps the MFMA operand reads free of bank conflicts.
-// MB (1..8) is the tile height in 32-row blocks: rows past the tile are
+// MB (2..8) is the tile height in 32-row blocks: rows past the tile are
 // neither loaded (beyond the MB blocks) nor multiplied.  The epilogue stages
 // the output tile in LDS and writes whole rows with 16-byte stores.
 //
@@ -673,7 +698,7 @@ __device__ __forceinline__ void gemm_tile(const GemmTile& t, uint8_t* smem,
   }
 }
 
-template <bool GATEUP>
+template <bool GATEUP, bool V4>
 __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
     aima_moe_layer L, const uint16_t* __restrict__ src, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ tile_count, const int32_t* __restrict__ token_map,
@@ -684,6 +709,25 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
   const int slot = p >> 3;
   const int mt = (slot / ntiles_n) * 8 + (p & 7);
   if (mt >= *tile_count) return;
+
+  // Tiles of one 32-row block: their time is the dequantization of weights
+  // that feed a single MFMA each, so they take the integer operands of
+  // thin_tile.  Against f16 operands on this block's own path (T = 777,
+  // uniform routing): 192 against 213 us per call; T = 900, skewed: 140
+  // against 159; T = 2048, skewed (101 of 141 experts have at most 32 rows):
+  // 238 against 252.
+  if (tiles[4 * mt + 2] <= 32) {
+    const ThinArgs a{src, tiles, tile_count, token_map, row_weight, A, ntiles_n,
+                     act_out, contrib_out, cap.act32, cap.contrib32};
+    const int e = tiles[4 * mt + 0], rows = tiles[4 * mt + 2];
+    const int64_t row0 = tiles[4 * mt + 1];
+    if (rows <= 16) {
+      thin_tile<GATEUP, 1, kThinTurn, V4, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
+    } else {
+      thin_tile<GATEUP, 2, kThinTurn, V4, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
+    }
+    return;
+  }
 
   GemmTile t;
   t.ntile = slot % ntiles_n;
@@ -751,7 +795,6 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
   }
 
   switch ((t.rows + 31) >> 5) {
-    case 1: gemm_tile<GATEUP, 1>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
     case 2: gemm_tile<GATEUP, 2>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
     case 3: gemm_tile<GATEUP, 3>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
     case 4: gemm_tile<GATEUP, 4>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
@@ -1002,8 +1045,8 @@ static int launch_schedule(const int32_t* ids, int stride, const float* weights,
   int rc = launch_check("grouped schedule count");
   if (rc != AIMA_OK) return rc;
   hipLaunchKernelGGL(sched_scan_kernel, dim3(1), dim3(1024), 0, st, w.block_base, (int32_t)d.nb,
-                     d.E, Ep, (int32_t)d.T, (int32_t)d.A, with_shared ? 1 : 0, w.offsets, w.tiles,
-                     w.tile_count);
+                     d.E, Ep, (int32_t)d.T, (int32_t)d.A, with_shared ? 1 : 0, d.bm_log2, w.offsets,
+                     w.tiles, w.tile_count);
   rc = launch_check("grouped schedule scan");
   if (rc != AIMA_OK) return rc;
   hipLaunchKernelGGL(sched_scatter_kernel, dim3((unsigned)d.nb), dim3(kSchedBlock), 0, st, ids,
@@ -1025,6 +1068,51 @@ static int record(hipEvent_t e, hipStream_t st) {
   return e ? hip_check(hipEventRecord(e, st), "hipEventRecord(prefill stage)") : AIMA_OK;
 }
 
+// Whether a turn's scales and zero points of a row can be loaded as vectors:
+// whole turns along K, every row's run aligned.
+static bool thin_vectors(int64_t K, const aima_u4_tensor* const (&w)[4]) {
+  bool ok = K % (128 * kThinTurn) == 0;
+  for (const aima_u4_tensor* t : w) ok = ok && aligned(t->scale, 8) && aligned(t->zp, 2);
+  return ok;
+}
+
+// One grouped GEMM of the layer over the schedule's tiles: 16-row tiles in
+// blocks of 256 threads, 256-row tiles in blocks of 512 (tile_rows_log2).
+template <bool GATEUP>
+static int launch_gemm(const aima_moe_layer& L, const uint16_t* src, const PrefillDims& d,
+                       const PrefillWs& w, const GemmCapture& cap, hipStream_t st) {
+  const int64_t K = GATEUP ? d.H : d.I;
+  const aima_u4_tensor* const tensors[4] = {GATEUP ? &L.gate_up : &L.down,
+                                            GATEUP ? &L.shared_gate_up : &L.shared_down,
+                                            GATEUP ? &L.up : &L.down,
+                                            GATEUP ? &L.shared_up : &L.shared_down};
+  const bool v4 = thin_vectors(K, tensors);
+  const unsigned mtiles = (unsigned)round_up(d.max_tiles, 8);
+  if (d.bm_log2 == kMinTileLog2) {
+    const int nt = GATEUP ? d.I / 64 : d.H / 128;
+    const ThinArgs a{src,   w.tiles,   w.tile_count, w.token_map, w.row_weight, d.A, nt,
+                     w.act, w.contrib, cap.act32,    cap.contrib32};
+    const dim3 grid(mtiles * nt), block(kThinThreads);
+    const size_t lds = thin_lds_bytes(1, kThinTurn, K / 128);
+    if (v4) {
+      hipLaunchKernelGGL((grouped_thin_kernel<GATEUP, true>), grid, block, lds, st, L, a);
+    } else {
+      hipLaunchKernelGGL((grouped_thin_kernel<GATEUP, false>), grid, block, lds, st, L, a);
+    }
+  } else {
+    const int nt = GATEUP ? d.I / 128 : d.H / 256;
+    const dim3 grid(mtiles * nt), block(kGemmThreads);
+    if (v4) {
+      hipLaunchKernelGGL((grouped_gemm_kernel<GATEUP, true>), grid, block, 0, st, L, src, w.tiles,
+                         w.tile_count, w.token_map, w.row_weight, d.A, nt, w.act, w.contrib, cap);
+    } else {
+      hipLaunchKernelGGL((grouped_gemm_kernel<GATEUP, false>), grid, block, 0, st, L, src, w.tiles,
+                         w.tile_count, w.token_map, w.row_weight, d.A, nt, w.act, w.contrib, cap);
+    }
+  }
+  return launch_check(GATEUP ? "grouped gate/up GEMM" : "grouped down GEMM");
+}
+
 // sigma_in: the shared-expert gate per token if already known (null: the
 // combine computes it from x); next: fusion of the next layer's input.
 static int prefill_layer(const aima_moe_layer& L, const uint16_t* x, const uint16_t* residual,
@@ -1037,23 +1125,10 @@ static int prefill_layer(const aima_moe_layer& L, const uint16_t* x, const uint1
   rc = launch_schedule(ids, call.stride ? call.stride : d.k, weights, d, w, !call.routed_f32, st);
   if (rc != AIMA_OK) return rc;
   if ((rc = record(call.ev[1], st)) != AIMA_OK) return rc;
-  const unsigned mtiles = (unsigned)round_up(d.max_tiles, 8);
-  {
-    const int nt = d.I / 128;
-    hipLaunchKernelGGL((grouped_gemm_kernel<true>), dim3(mtiles * nt), dim3(kGemmThreads), 0, st,
-                       L, x, w.tiles, w.tile_count, w.token_map, w.row_weight, d.A, nt, w.act,
-                       w.contrib, call.cap);
-  }
-  rc = launch_check("grouped gate/up GEMM");
+  rc = launch_gemm<true>(L, x, d, w, call.cap, st);
   if (rc != AIMA_OK) return rc;
   if ((rc = record(call.ev[2], st)) != AIMA_OK) return rc;
-  {
-    const int nt = d.H / 256;
-    hipLaunchKernelGGL((grouped_gemm_kernel<false>), dim3(mtiles * nt), dim3(kGemmThreads), 0, st,
-                       L, w.act, w.tiles, w.tile_count, w.token_map, w.row_weight, d.A, nt, w.act,
-                       w.contrib, call.cap);
-  }
-  rc = launch_check("grouped down GEMM");
+  rc = launch_gemm<false>(L, w.act, d, w, call.cap, st);
   if (rc != AIMA_OK) return rc;
   if ((rc = record(call.ev[3], st)) != AIMA_OK) return rc;
   if (call.routed_f32) {

@@ -270,3 +270,36 @@ def test_prefill_largest_batch(pkg, dev, layer_full):
                                 w[sel].cpu().numpy(), threads=THREADS)
     assert_parity(got, ref, what="largest batch")
     del out, x
+
+
+@pytest.mark.parametrize("H,I", [(512, 512), (512, 128), (768, 384)])
+@pytest.mark.parametrize("experts", [96, 16])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_prefill_thin_tiles(pkg, dev, H, I, experts, shift):
+    """Tiles at the edges of the thin-tile path (1, 15, 16, 17, 31, 32 rows),
+    one row above it (33) and a full tile with a one-row remainder, in 16-row
+    tiles (96 experts: at most 10 rows per expert) and 256-row ones (16).  K of
+    1, 3, 4 and 6 quantization groups, and scales and zero points off their
+    vector alignment (shift), cover both ways of loading them.  f16 operands
+    and intermediates: 2e-3, as the other prefill tests."""
+    layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=experts, seed=300 + H + I, device=dev)
+    mw = moe_to_oracle(layer)
+    if shift:
+        def off(t):
+            flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)
+            flat[1:] = t.reshape(-1)
+            return flat[1:].reshape(t.shape)
+
+        for w in (layer.gate_up, layer.down, layer.shared_gate_up, layer.shared_down):
+            w.scale, w.zp = off(w.scale), off(w.zp)
+    counts = [1, 15, 16, 17, 31, 32, 33] if experts == 96 else [1, 15, 16, 17, 31, 32, 33, 257]
+    ids = np.repeat(np.arange(len(counts)) * (experts // len(counts)), counts).astype(np.int32)
+    ids = np.random.default_rng(H + I).permutation(ids)[:, None].copy()
+    T = len(ids)
+    assert (T <= 10 * experts) == (experts == 96)
+    x = pkg.synth.activations(T, H, 301, dev)
+    w = torch.ones((T, 1), device=dev)
+    out = pkg.grouped_moe_prefill(layer, x, torch.from_numpy(ids).to(dev), w)
+    torch.cuda.synchronize()
+    ref = oracle.moe_ffn_tokens(mw, f16_to_f32(x), ids, w.cpu().numpy(), threads=THREADS)
+    assert_parity(f16_to_f32(out), ref, what=f"thin tiles H={H} I={I} E={experts}")
