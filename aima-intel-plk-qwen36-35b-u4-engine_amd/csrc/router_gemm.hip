@@ -5,14 +5,8 @@
 //
 // logits[T][E] = X[T][H] . W[E][H]^T in f32 (2 T E H flops: 2.1 GFLOP at
 // T = 2048, E = 256, H = 2048) on the f32 matrix cores
-// (v_mfma_f32_32x32x2_f32: f32 operands, f32 accumulation).  A block of 8
-// waves owns a 64-token x 64-expert tile; wave w computes the 32 x 32
-// quarter w % 4 over the K half w / 4, and the two K halves are added
-// through LDS (half 0 + half 1, the same order every call).  Each lane
-// loads 4 consecutive k of its token row and of its expert row with one
-// 16-byte load per 8 k: MFMA j of the 4 per step then sees k0 + 4 h + j in
-// lane half h, for both operands, so the 8 k of a step are each summed once.
-// An f16 input is first widened to f32 in the caller's workspace.
+// (v_mfma_f32_32x32x2_f32: f32 operands, f32 accumulation).  An f16 input is
+// widened in registers.
 #include "common.h"
 
 namespace aima {
@@ -25,54 +19,186 @@ namespace {
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kRgThreads = 512;
-constexpr int kRgTile = 64;  // tokens and experts per block
+constexpr int kRgWaves = 8;
+constexpr int kRgThreads = 64 * kRgWaves;
+constexpr int kRgChunk = 128;  // k per step
 
-__global__ __launch_bounds__(256) void widen_f16_kernel(const uint16_t* __restrict__ in,
-                                                        float* __restrict__ out, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) out[i] = h2f(in[i]);
+// 8 consecutive values of a row in LDS as f32 (row: its chunk, 16-byte piece
+// p at slot p ^ (row index % pieces); k0: first value)
+__device__ __forceinline__ void rg_read(const float* row, int swz, int k0, float (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const u32x4 d = *reinterpret_cast<const u32x4*>(row + (((k0 / 4 + i) ^ swz) * 4));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[4 * i + j] = as_f32(d[j]);
+  }
+}
+__device__ __forceinline__ void rg_read(const uint16_t* row, int swz, int k0, float (&v)[8]) {
+  const u32x4 d = *reinterpret_cast<const u32x4*>(row + (((k0 / 8) ^ (swz & 15)) * 8));
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t w = d[j];
+    v[2 * j] = h2f((uint16_t)(w & 0xffffu));
+    v[2 * j + 1] = h2f((uint16_t)(w >> 16));
+  }
 }
 
+// A block of 8 waves owns 32 NA tokens x 32 experts.  K runs in steps of 128
+// through two LDS buffers (the next step's rows are loaded into registers
+// while this one is multiplied); wave w multiplies k 16 w .. 16 w + 15 of
+// every step, lane half h the 8 from 8 h (MFMA j sees k0 + 8 h + j in both
+// operands), and the eight partial tiles are added through LDS in wave order,
+// the same every call.
+//
+// Bound: the f32 MFMAs (13 us at the 163 TFLOP/s peak for T = 2048, E = 256,
+// H = 2048).  The output has only 512 32 x 32 tiles there, two per CU: K split
+// over the waves of a block fills the chip.  Rows read straight into the
+// operands' lanes (32 rows per load) made T = 4096 f32 88 us a call with its
+// selection, against 57 to 61 here; 64 x 64 tiles with two K halves, read the
+// same way, took 68 us at T = 2048 where this takes 28 (f16 input).
+// Blocks are mapped XCD-aware: a token tile's expert blocks run on one XCD.
+//
 // Rows past T (tokens) or E (experts) load the last row (valid memory) and
-// are never stored.  H % 16 == 0 and both matrices 16-byte aligned (checked
-// on the host).
-__global__ __launch_bounds__(kRgThreads) void router_gemm_kernel(
-    const float* __restrict__ x, const float* __restrict__ w, int64_t T, int E, int H,
+// are never stored; k past H load as zeros.  H % 16 == 0 and both matrices
+// 16-byte aligned (checked on the host).
+template <typename X, int NA>
+__global__ __launch_bounds__(kRgThreads, 2) void router_gemm_kernel(
+    const X* __restrict__ x, const float* __restrict__ w, int64_t T, int E, int H, int ey,
     float* __restrict__ logits) {
-  __shared__ float part[4][16][64];  // K-half 1 partial sums, [quarter][acc][lane]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int q = wave & 3, kh = wave >> 2;
-  const int64_t t0 = (int64_t)blockIdx.x * kRgTile + 32 * (q >> 1);
-  const int e0 = (int)blockIdx.y * kRgTile + 32 * (q & 1);
-  const int64_t tr = t0 + (lane & 31) < T ? t0 + (lane & 31) : T - 1;
-  const int er = e0 + (lane & 31) < E ? e0 + (lane & 31) : E - 1;
-  const int half = H / 2;
-  const float* xp = x + tr * H + kh * half + 4 * (lane >> 5);
-  const float* wp = w + (int64_t)er * H + kh * half + 4 * (lane >> 5);
-  f32x16_t acc = f32x16_t{};
-  for (int k = 0; k < half; k += 8) {
-    const float4 a = *reinterpret_cast<const float4*>(xp + k);
-    const float4 b = *reinterpret_cast<const float4*>(wp + k);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
-  }
-  if (kh == 1) {
+  constexpr int kXVals = 16 / sizeof(X);         // values of a 16-byte piece
+  constexpr int kXPieces = kRgChunk / kXVals;    // pieces of a token row's step
+  constexpr int kWPieces = kRgChunk / 4;
+  constexpr int kXPer = NA * 32 * kXPieces / kRgThreads, kWPer = 32 * kWPieces / kRgThreads;
+  constexpr int kXBytes = NA * 32 * kRgChunk * sizeof(X), kWBytes = 32 * kRgChunk * 4;
+  constexpr int kPartBytes = kRgWaves * NA * 16 * 64 * 4;
+  constexpr int kSmem = 2 * (kXBytes + kWBytes) > kPartBytes ? 2 * (kXBytes + kWBytes) : kPartBytes;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kSmem];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int p = blockIdx.x, slot = p >> 3;
+  const int64_t t0 = (int64_t)((slot / ey) * 8 + (p & 7)) * (32 * NA);
+  const int e0 = (slot % ey) * 32;
+  if (t0 >= T) return;
+
+  const X* xp[kXPer];
+  const float* wp[kWPer];
+  const int xk = (tid % kXPieces) * kXVals, wk = (tid % kWPieces) * 4;
+  const int xr = tid / kXPieces, wr = tid / kWPieces;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) part[q][i][lane] = acc[i];
+  for (int i = 0; i < kXPer; ++i) {
+    const int64_t t = t0 + xr + i * (kRgThreads / kXPieces);
+    xp[i] = x + (t < T ? t : T - 1) * H + xk;
   }
+#pragma unroll
+  for (int i = 0; i < kWPer; ++i) {
+    const int e = e0 + wr + i * (kRgThreads / kWPieces);
+    wp[i] = w + (int64_t)(e < E ? e : E - 1) * H + wk;
+  }
+  struct Regs {
+    u32x4 x[kXPer], w[kWPer];
+  };
+  auto load = [&](int k, Regs& d) {
+    const bool xin = k + xk < H, win = k + wk < H;  // whole pieces: H % 16 == 0
+    const int xo = xin ? k : -xk, wo = win ? k : -wk;
+#pragma unroll
+    for (int i = 0; i < kXPer; ++i) {
+      d.x[i] = *reinterpret_cast<const u32x4*>(xp[i] + xo);
+      d.x[i] = xin ? d.x[i] : u32x4{};
+    }
+#pragma unroll
+    for (int i = 0; i < kWPer; ++i) {
+      d.w[i] = *reinterpret_cast<const u32x4*>(wp[i] + wo);
+      d.w[i] = win ? d.w[i] : u32x4{};
+    }
+  };
+  auto store = [&](const Regs& d, uint8_t* buf) {
+#pragma unroll
+    for (int i = 0; i < kXPer; ++i) {
+      const int r = xr + i * (kRgThreads / kXPieces);
+      *reinterpret_cast<u32x4*>(buf + (r * kXPieces + ((tid % kXPieces) ^ (r & (kXPieces - 1)))) * 16) =
+          d.x[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kWPer; ++i) {
+      const int r = wr + i * (kRgThreads / kWPieces);
+      *reinterpret_cast<u32x4*>(buf + kXBytes +
+                                (r * kWPieces + ((tid % kWPieces) ^ (r & (kWPieces - 1)))) * 16) = d.w[i];
+    }
+  };
+
+  f32x16_t acc[NA];
+#pragma unroll
+  for (int a = 0; a < NA; ++a) acc[a] = f32x16_t{};
+  const int row = lane & 31, k0 = 16 * wave + 8 * (lane >> 5);
+  auto multiply = [&](const uint8_t* buf) {
+    float b[8], av[NA][8];
+    rg_read(reinterpret_cast<const float*>(buf + kXBytes) + row * kRgChunk, row, k0, b);
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+      rg_read(reinterpret_cast<const X*>(buf) + (32 * a + row) * kRgChunk, row, k0, av[a]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+        acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[a][j], b[j], acc[a], 0, 0, 0);
+    }
+  };
+  // two steps of rows in flight: a step's loads have the next two
+  // multiplications to land
+  uint8_t* const buf0 = smem;
+  uint8_t* const buf1 = smem + kXBytes + kWBytes;
+  Regs r0, r1;
+  load(0, r0);
+  load(kRgChunk, r1);
+  store(r0, buf0);
   __syncthreads();
-  if (kh == 1) return;
-  // lane l holds expert e0 + l % 32 of token rows 8 (i / 4) + 4 (l / 32) + i % 4
-  const int e = e0 + (lane & 31);
+  for (int k = 0; k < H; k += 2 * kRgChunk) {
+    load(k + 2 * kRgChunk, r0);
+    multiply(buf0);
+    store(r1, buf1);  // zeros past K
+    __syncthreads();
+    load(k + 3 * kRgChunk, r1);
+    multiply(buf1);
+    store(r0, buf0);
+    __syncthreads();
+  }
+
+  // partial tiles [wave][frag][acc][lane]; every wave adds its share of them
+  float* part = reinterpret_cast<float*>(smem);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int64_t t = t0 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-    const float v = acc[i] + part[q][i][lane];
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part[((wave * NA + a) * 16 + i) * 64 + lane] = acc[a][i];
+  __syncthreads();
+#pragma unroll
+  for (int f = 0; f < 2 * NA; ++f) {
+    const int c = wave * 2 * NA + f, a = c >> 4, i = c & 15;
+    float v = part[c * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < kRgWaves; ++q) v += part[(q * NA * 16 + c) * 64 + lane];
+    // lane l holds expert e0 + l % 32 of token rows 8 (i / 4) + 4 (l / 32) + i % 4
+    const int64_t t = t0 + 32 * a + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    const int e = e0 + (lane & 31);
     if (t < T && e < E) logits[t * E + e] = v;
   }
+}
+
+// 64 tokens per block (fewer reads of the router's rows) once that leaves
+// more than one block per CU: T = 2048, E = 256 (256 such blocks) 35.3 us a
+// call against 33.3 in 512 blocks of 32 tokens; T = 4096, f16: 52.6 against
+// 55.5 (f32: 61.4 against 56.8).
+template <typename X>
+int router_gemm_launch(const X* x, int64_t tokens, int experts, int64_t hidden, const float* w,
+                       float* logits, hipStream_t st) {
+  const int ey = (experts + 31) / 32;
+  const int64_t wide = (tokens + 63) / 64, narrow = (tokens + 31) / 32;
+  if (wide * ey > 256) {
+    hipLaunchKernelGGL((router_gemm_kernel<X, 2>), dim3((unsigned)(round_up(wide, 8) * ey)),
+                       dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, ey, logits);
+  } else {
+    hipLaunchKernelGGL((router_gemm_kernel<X, 1>), dim3((unsigned)(round_up(narrow, 8) * ey)),
+                       dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, ey, logits);
+  }
+  return launch_check("router_gemm");
 }
 
 size_t router_ws_bytes(int64_t tokens, int64_t hidden, int input_f32) {
@@ -109,27 +235,15 @@ extern "C" int aima_router_gemm_topk(const void* hidden_states, int32_t input_f3
                "router_gemm_topk: k must be in [1, min(16, experts)]");
   AIMA_REQUIRE(min_weight_sum > 0.f, "router_gemm_topk: minimum weight sum must be positive");
   const hipStream_t st = (hipStream_t)stream;
-  const float* x = static_cast<const float*>(hidden_states);
-  if (!input_f32) {
-    AIMA_REQUIRE(workspace && aligned(workspace, 256) &&
-                     workspace_bytes >= router_ws_bytes(tokens, hidden, 0),
-                 "router_gemm_topk: an f16 input needs the workspace");
-    float* wide = reinterpret_cast<float*>(static_cast<char*>(workspace) + kWsHeader);
-    const int64_t n = tokens * hidden;
-    hipLaunchKernelGGL(widen_f16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(hidden_states), wide, n);
-    const int rc = launch_check("router_gemm widen");
-    if (rc != AIMA_OK) return rc;
-    x = wide;
-  }
-  {
-    const dim3 grid((unsigned)((tokens + kRgTile - 1) / kRgTile),
-                    (unsigned)((experts + kRgTile - 1) / kRgTile));
-    hipLaunchKernelGGL(router_gemm_kernel, grid, dim3(kRgThreads), 0, st, x, router_weight,
-                       tokens, experts, (int)hidden, logits);
-    const int rc = launch_check("router_gemm");
-    if (rc != AIMA_OK) return rc;
-  }
+  // (an f16 input was once widened there; the size a caller queries stays)
+  AIMA_REQUIRE(input_f32 || (workspace && aligned(workspace, 256) &&
+                             workspace_bytes >= router_ws_bytes(tokens, hidden, 0)),
+               "router_gemm_topk: an f16 input needs the workspace");
+  const int rc = input_f32 ? router_gemm_launch(static_cast<const float*>(hidden_states), tokens,
+                                                experts, hidden, router_weight, logits, st)
+                           : router_gemm_launch(static_cast<const uint16_t*>(hidden_states), tokens,
+                                                experts, hidden, router_weight, logits, st);
+  if (rc != AIMA_OK) return rc;
   return router_topk_launch(logits, tokens, experts, k, min_weight_sum, ids, weights, st,
                             nullptr);
 }

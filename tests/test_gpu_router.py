@@ -25,9 +25,8 @@ def _router(E, H, seed, dev):
                                      (2048, 256, 8, 2048), (77, 16, 4, 2048),
                                      (33, 100, 8, 528)])
 def test_router_gemm_topk(pkg, dev, T, E, k, H):
-    """Tiles of 64 tokens x 64 experts: partial tiles in both dimensions
-    (T = 1, 33, 77, 300; E = 16, 100) and a hidden size whose K halves are
-    not a multiple of the 64-wide steps (528)."""
+    """Partial tiles in both dimensions (T = 1, 33, 77, 300; E = 16, 100) and
+    a hidden size that is no multiple of the K steps (528)."""
     x = pkg.synth.activations(T, H, T + E, dev).float()
     W = _router(E, H, T + 1, dev)
     ids, w, logits = pkg.router_gemm_topk(x, W, k)
@@ -36,6 +35,27 @@ def test_router_gemm_topk(pkg, dev, T, E, k, H):
     got = logits.cpu().numpy()
     assert np.abs(got - ref).max() <= 1e-5 * np.abs(ref).max()
     ref_ids, ref_w = oracle.router_topk_tokens(got, k)
+    assert np.array_equal(ids.cpu().numpy(), ref_ids)
+    assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")
+
+
+@pytest.mark.parametrize("T,E,H", [(31, 33, 16), (33, 32, 144), (65, 64, 384),
+                                   (16449, 17, 272)])
+@pytest.mark.parametrize("f32", [True, False])
+def test_router_gemm_edges(pkg, dev, T, E, H, f32):
+    """Both block widths (16,449 tokens: 64-token blocks), partial blocks in
+    both dimensions, K below one 128-wide step, with a partial last step and
+    with an odd number of steps.  f32 sums of H products: each at most
+    H * 2^-24 of the sum of its terms' magnitudes off."""
+    x = pkg.synth.activations(T, H, T + H, dev)
+    x = x.float() if f32 else x
+    W = _router(E, H, T + 2, dev)
+    ids, w, logits = pkg.router_gemm_topk(x, W, 4)
+    torch.cuda.synchronize()
+    ref = x.double() @ W.double().T
+    bound = (x.double().abs() @ W.double().abs().T) * H * 2.0 ** -24
+    assert bool(((logits.double() - ref).abs() <= bound).all())
+    ref_ids, ref_w = oracle.router_topk_tokens(logits.cpu().numpy(), 4)
     assert np.array_equal(ids.cpu().numpy(), ref_ids)
     assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")
 
