@@ -121,7 +121,7 @@ __device__ __forceinline__ float as_f32_value(float v) {
   return v;
 }
 
-template <bool GATEUP, int NB, int CH, bool V4, int TH>
+template <bool GATEUP, int NB, int CH, bool V4, bool CAP, int TH>
 __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_layer& L, uint8_t* smem,
                                           int e, int64_t row0, int rows, int ntile) {
   static_assert(kThinTurn % CH == 0 && CH % 2 == 0, "whole token chunks per turn");
@@ -329,14 +329,14 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
         const float g = acc[0][b][j] * 16777216.0f, u = acc[1][b][j] * 16777216.0f;
         const float o = as_f32_value(g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g)));
         stage[m * (kCols + 8) + n] = f2h(o);
-        if (a.act32 && m < rows) a.act32[(row0 + m) * ld + col0 + n] = o;
+        if (CAP && a.act32 && m < rows) a.act32[(row0 + m) * ld + col0 + n] = o;
       } else {
         const float wt = routed && m < rows ? a.row_weight[row0 + m] : 1.0f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const float o = as_f32_value(wt * (acc[h][b][j] * 16777216.0f));
           stage[m * (kCols + 8) + 16 * h + n] = f2h(o);
-          if (a.contrib32 && m < rows) a.contrib32[(row0 + m) * ld + col0 + 16 * h + n] = o;
+          if (CAP && a.contrib32 && m < rows) a.contrib32[(row0 + m) * ld + col0 + 16 * h + n] = o;
         }
       }
     }
@@ -358,7 +358,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
 // loads and epilogue pass under another's stream (blocks of 512 threads:
 // T = 96 119 against 108 us per call).  Blocks are mapped XCD-aware, as in
 // grouped_gemm_kernel: tile i on XCD i % 8, its blocks consecutive there.
-template <bool GATEUP, bool V4>
+template <bool GATEUP, bool V4, bool CAP>
 __global__ __launch_bounds__(kThinThreads, V4 ? 3 : 2) void grouped_thin_kernel(aima_moe_layer L,
                                                                                 ThinArgs a) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t thin_smem[];
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(kThinThreads, V4 ? 3 : 2) void grouped_thin_kernel(
   const int slot = p >> 3;
   const int mt = (slot / a.ntiles_n) * 8 + (p & 7);
   if (mt >= *a.tile_count) return;
-  thin_tile<GATEUP, 1, kThinTurn, V4, kThinThreads>(a, L, thin_smem, a.tiles[4 * mt + 0],
+  thin_tile<GATEUP, 1, kThinTurn, V4, CAP, kThinThreads>(a, L, thin_smem, a.tiles[4 * mt + 0],
                                                     a.tiles[4 * mt + 1], a.tiles[4 * mt + 2],
                                                     slot % a.ntiles_n);
 }

@@ -77,7 +77,9 @@ static int64_t tile_bound(const PrefillDims& d, int64_t bm) {
 // Beyond, an expert's weights are read once per 16 rows for nothing: at 12.5
 // per expert 141 against 160 us if the routing is uniform, but 116 against
 // 109 if it is skewed, 14 per expert 124 against 110.
-static int tile_rows_log2(const PrefillDims& d) { return d.A <= 10 * (int64_t)d.E ? 4 : 8; }
+static int tile_rows_log2(const PrefillDims& d) {
+  return d.A <= 10 * (int64_t)d.E ? kMinTileLog2 : 8;
+}
 
 static PrefillDims prefill_dims(const aima_moe_layer* L, int64_t T, int k) {
   PrefillDims d;
@@ -483,7 +485,7 @@ struct GemmCapture {
   float* contrib32;  // [rows][H]
 };
 
-template <bool GATEUP, int MB>
+template <bool GATEUP, int MB, bool CAP>
 __device__ __forceinline__ void gemm_tile(const GemmTile& t, uint8_t* smem,
                                           const aima_moe_layer& L,
                                           const float* __restrict__ row_weight,
@@ -536,15 +538,14 @@ __device__ __forceinline__ void gemm_tile(const GemmTile& t, uint8_t* smem,
 
   // sA: the group's token rows in LDS, row m at sA + 256 m
   auto compute = [&](int g, const uint8_t* sA, const WGroup& w) {
-    const uint32_t z = (w.z >> (((t.zbase + g) & 1) * 4)) & 0xfu;
     const f16x2 ss2 = u4_ss2(w.s);
-    const f16x2 zz2 = u4_zz2(z);
+    const f16x2 zz2 = u4_zz2((w.z >> (((t.zbase + g) & 1) * 4)) & 0xfu);
     auto bfrag = [&](int mb, int j) {
       const int m = mb * 32 + n;
       const int slot = (hh * 8 + j) ^ (m & 15);
       return *reinterpret_cast<const f16x8*>(sA + m * 256 + slot * 16);
     };
-    auto wword = [&](int j) { return j < 4 ? w.q0[j & 3] : w.q1[j & 3]; };
+    auto operand = [&](int j) { return dequant8(j < 4 ? w.q0[j & 3] : w.q1[j & 3], zz2, ss2, magic); };
     // Software pipeline over the 8 k-steps: step j issues the operand reads
     // and the dequantization of step j+1, then its MB independent MFMAs (one
     // per accumulator).  The scheduling fences keep each step's MFMAs
@@ -554,22 +555,20 @@ __device__ __forceinline__ void gemm_tile(const GemmTile& t, uint8_t* smem,
     f16x8 a[2];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) bf[0][mb] = bfrag(mb, 0);
-    a[0] = dequant8(wword(0), zz2, ss2, magic);
+    a[0] = operand(0);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if (j + 1 < 8) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) bf[(j + 1) & 1][mb] = bfrag(mb, j + 1);
-        a[(j + 1) & 1] = dequant8(wword(j + 1), zz2, ss2, magic);
+        a[(j + 1) & 1] = operand(j + 1);
       }
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
+      for (int mb = 0; mb < MB; ++mb)
         acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j & 1], bf[j & 1][mb], acc[mb], 0, 0, 0);
-      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-
 
   const int GK = t.GK;
   constexpr int kResidentGroupBytes = MB * 32 * 256;  // token rows of one group
@@ -649,7 +648,7 @@ __device__ __forceinline__ void gemm_tile(const GemmTile& t, uint8_t* smem,
         v.y = pack_h2(a[2], a[3]);
         const int chunk = (wave * 2 + q) ^ (m & (kChunks - 1));
         *reinterpret_cast<u32x2*>(rowp + chunk * 16 + hh * 8) = v;
-        if (cap.act32 && m < t.rows) {
+        if (CAP && cap.act32 && m < t.rows) {
           *reinterpret_cast<float4*>(cap.act32 + (t.row0 + m) * I + col_base + (wave * 2 + q) * 8) =
               make_float4(a[0], a[1], a[2], a[3]);
         }
@@ -665,7 +664,7 @@ __device__ __forceinline__ void gemm_tile(const GemmTile& t, uint8_t* smem,
         v.y = pack_h2(o[2], o[3]);
         const int chunk = (wave * 4 + q) ^ (m & (kChunks - 1));
         *reinterpret_cast<u32x2*>(rowp + chunk * 16 + hh * 8) = v;
-        if (cap.contrib32 && m < t.rows) {
+        if (CAP && cap.contrib32 && m < t.rows) {
           *reinterpret_cast<float4*>(cap.contrib32 + (t.row0 + m) * H + col_base + (wave * 4 + q) * 8) =
               make_float4(o[0], o[1], o[2], o[3]);
         }
@@ -698,7 +697,7 @@ __device__ __forceinline__ void gemm_tile(const GemmTile& t, uint8_t* smem,
   }
 }
 
-template <bool GATEUP, bool V4>
+template <bool GATEUP, bool V4, bool CAP>
 __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
     aima_moe_layer L, const uint16_t* __restrict__ src, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ tile_count, const int32_t* __restrict__ token_map,
@@ -722,9 +721,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
     const int e = tiles[4 * mt + 0], rows = tiles[4 * mt + 2];
     const int64_t row0 = tiles[4 * mt + 1];
     if (rows <= 16) {
-      thin_tile<GATEUP, 1, kThinTurn, V4, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
+      thin_tile<GATEUP, 1, kThinTurn, V4, CAP, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
     } else {
-      thin_tile<GATEUP, 2, kThinTurn, V4, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
+      thin_tile<GATEUP, 2, kThinTurn, V4, CAP, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
     }
     return;
   }
@@ -795,13 +794,245 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
   }
 
   switch ((t.rows + 31) >> 5) {
-    case 2: gemm_tile<GATEUP, 2>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
-    case 3: gemm_tile<GATEUP, 3>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
-    case 4: gemm_tile<GATEUP, 4>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
-    case 5: gemm_tile<GATEUP, 5>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
-    case 6: gemm_tile<GATEUP, 6>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
-    case 7: gemm_tile<GATEUP, 7>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
-    default: gemm_tile<GATEUP, 8>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+    case 2: gemm_tile<GATEUP, 2, CAP>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+    case 3: gemm_tile<GATEUP, 3, CAP>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+    case 4: gemm_tile<GATEUP, 4, CAP>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+    case 5: gemm_tile<GATEUP, 5, CAP>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+    case 6: gemm_tile<GATEUP, 6, CAP>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+    case 7: gemm_tile<GATEUP, 7, CAP>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+    default: gemm_tile<GATEUP, 8, CAP>(t, smem, L, row_weight, act_out, contrib_out, cap); break;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// down GEMM with the tile's token rows resident
+// ---------------------------------------------------------------------------
+// K = inter <= 512: 128 token rows of a tile fit in LDS for the whole K
+// (128 KB).  A block of 8 waves loads them once and computes a range of
+// output columns against them, 64 columns of a wave at a time (two 32-row MFMA
+// operands, so each token operand read from LDS feeds two MFMAs).  After the
+// rows are in, the waves share nothing: no barriers, each streams its own
+// weights and writes its own outputs through 4 KB of LDS, so one wave's
+// dequantization and epilogue pass under another's MFMAs.
+//
+// Bound: with 4 K groups a tile's fixed costs weigh as much as its MFMAs.  Of
+// a 16-chunk block's ~40 us, ~6 load the rows, 2 x 4 groups take 2.3-2.9 each
+// (2.05 at the matrix cores' rate) and two epilogues ~2.5 each (the chip's
+// write bandwidth while all blocks store).  Loading only the first group's
+// rows before multiplying measured 3 % slower, one barrier-ringed kernel of
+// 4 waves x 64 weight rows, two blocks per CU, 6 %.  T = 16384 (hidden 2048,
+// inter 512): 427 us a layer, grouped_gemm_kernel 490 (same box; MFMA-bound
+// 270 at the rate of a large f16 product).
+constexpr int kDownRows = 128;
+constexpr int kDownMaxGroups = 4;
+constexpr int kDownTokens = kDownRows * kDownMaxGroups * 256;  // bytes of LDS
+constexpr int kDownChunk = 64;                                 // columns of a wave at a time
+
+struct DownTile {
+  int64_t row0;
+  int e, rows, GK, chunk0, chunks;  // first column chunk of this wave, end of the block's
+};
+
+template <int MB, bool CAP>
+__device__ __forceinline__ void down_tile(const DownTile& t, const aima_moe_layer& L,
+                                          const uint16_t* __restrict__ act,
+                                          const float* __restrict__ row_weight, uint8_t* smem,
+                                          uint16_t* __restrict__ contrib,
+                                          float* __restrict__ contrib32) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, hh = lane >> 5;
+  const int GK = t.GK;
+  const int64_t H = L.hidden, K = L.inter;
+  const bool routed = t.e < L.experts;
+  const aima_u4_tensor& W = routed ? L.down : L.shared_down;
+  const uint32_t lds0 = lds_addr(smem);
+  constexpr int kGroup = MB * 32 * 256;  // bytes of one group's rows
+
+  // token rows, as in gemm_tile: block instruction q = wave + 8 i covers rows
+  // 4 q .. 4 q + 3, piece p of row r in slot p ^ (r & 15)
+  const void* base = uniform_ptr(act);
+#pragma unroll
+  for (int g = 0; g < kDownMaxGroups; ++g) {
+    if (g < GK) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const int r = 4 * (wave + 8 * i) + (lane >> 4);
+        const int64_t grow = t.row0 + (r < t.rows ? r : 0);
+        const int piece = (lane & 15) ^ (r & 15);
+        lds_load16(base, (uint32_t)((grow * K + g * 128 + piece * 8) * 2),
+                   lds0 + (uint32_t)(g * kGroup + (wave + 8 * i) * 1024));
+      }
+    }
+  }
+
+  struct WGroup {
+    u32x4 q0, q1;
+    uint32_t s, z;
+  };
+  const int64_t e0 = routed ? (int64_t)t.e * H : 0;
+  const int64_t wstep = 32 * (K / 2), sstep = 32 * GK;  // to the second 32 columns
+  auto load_w = [&](int chunk, int g, WGroup (&r)[2]) {
+    const int64_t row = e0 + (int64_t)chunk * kDownChunk + n;
+    const uint8_t* wq = W.qweight + row * (K / 2) + hh * 32 + g * 64;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      const int64_t at = row * GK + f * sstep + g;
+      r[f].q0 = gload16(wq + f * wstep);
+      r[f].q1 = gload16(wq + f * wstep + 16);
+      r[f].s = ((const AIMA_GLOBAL uint16_t*)W.scale)[at];
+      r[f].z = (uint32_t)((const AIMA_GLOBAL uint8_t*)W.zp)[at >> 1] >> ((at & 1) * 4);
+    }
+  };
+  float wt[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int m = mb * 32 + n;
+    wt[mb] = routed ? row_weight[t.row0 + (m < t.rows ? m : 0)] : 1.0f;
+  }
+  const uint32_t magic = u4_magic();
+  WGroup wn[2];
+  load_w(t.chunk0 < t.chunks ? t.chunk0 : 0, 0, wn);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  plain_barrier();
+
+  uint8_t* stage = smem + kDownTokens + wave * 4096;
+  const uint32_t out_off = (uint32_t)((lane >> 3) * H * 2 + (lane & 7) * 16);
+  for (int chunk = t.chunk0; chunk < t.chunks; chunk += 8) {
+    f32x16 acc[2][MB];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) acc[f][mb] = f32x16{};
+    for (int g = 0; g < GK; ++g) {
+      const WGroup w[2] = {wn[0], wn[1]};
+      {
+        // the next group, of the next chunk at the end (past the last: this one again)
+        const bool over = g + 1 == GK;
+        const int nc = over && chunk + 8 < t.chunks ? chunk + 8 : chunk;
+        load_w(nc, over ? 0 : g + 1, wn);
+      }
+      f16x2 ss2[2], zz2[2];
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        ss2[f] = u4_ss2(w[f].s);
+        zz2[f] = u4_zz2(w[f].z & 0xfu);
+      }
+      const uint8_t* sA = smem + g * kGroup;
+      auto bfrag = [&](int mb, int j) {
+        return *reinterpret_cast<const f16x8*>(sA + (mb * 32 + n) * 256 +
+                                               (((hh * 8 + j) ^ (n & 15)) * 16));
+      };
+      auto operand = [&](int f, int j) {
+        return dequant8(j < 4 ? w[f].q0[j & 3] : w[f].q1[j & 3], zz2[f], ss2[f], magic);
+      };
+      f16x8 bf[2][MB];
+      f16x8 a[2];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) bf[0][mb] = bfrag(mb, 0);
+      a[0] = operand(0, 0);
+      // half-steps (k-step j, columns f): the next half-step's weights are
+      // dequantized and the next k-step's tokens read beside MB independent
+      // MFMAs; the fences keep each half-step's MFMAs together (gemm_tile)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          if (f == 0 && j + 1 < 8) {
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) bf[(j + 1) & 1][mb] = bfrag(mb, j + 1);
+          }
+          if (f == 0) {
+            a[1] = operand(1, j);
+          } else if (j + 1 < 8) {
+            a[0] = operand(0, j + 1);
+          }
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+            acc[f][mb] =
+                __builtin_amdgcn_mfma_f32_32x32x16_f16(a[f], bf[j & 1][mb], acc[f][mb], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    // outputs, 32 token rows x 64 columns at a time: lane (n, hh) holds
+    // columns 32 f + 8 q + 4 hh .. +3 of token row n in acc[f][mb][4 q ..]
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int m = mb * 32 + n;
+      if (mb > 0) wave_lds_sync();
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float o[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) o[c] = wt[mb] * acc[f][mb][4 * q + c];
+          const u32x2 v{pack_h2(o[0], o[1]), pack_h2(o[2], o[3])};
+          *reinterpret_cast<u32x2*>(stage + n * 128 + (((f * 4 + q) ^ (n & 7)) * 16) + hh * 8) = v;
+          if (CAP && contrib32 && m < t.rows) {
+            *reinterpret_cast<float4*>(contrib32 + (t.row0 + m) * H + chunk * kDownChunk + f * 32 +
+                                       q * 8 + hh * 4) = make_float4(o[0], o[1], o[2], o[3]);
+          }
+        }
+      }
+      wave_lds_sync();
+      char* out = reinterpret_cast<char*>(contrib + (t.row0 + mb * 32) * H + chunk * kDownChunk);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 8 * i + (lane >> 3), c = lane & 7;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(stage + r * 128 + ((c ^ (r & 7)) * 16));
+        if (mb * 32 + r < t.rows) {
+          // read once, by the combine: nontemporal
+          __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out + 16 * i * H + out_off));
+        }
+      }
+    }
+    wave_lds_sync();
+  }
+}
+
+// Grid: per tile of up to 256 rows, two halves of 128 rows and `splits`
+// column ranges of `cpb` chunks, consecutive on one XCD.
+template <bool V4, bool CAP>
+__global__ __launch_bounds__(512, 2) void grouped_down_kernel(
+    aima_moe_layer L, const uint16_t* __restrict__ act, const int32_t* __restrict__ tiles,
+    const int32_t* __restrict__ tile_count, const float* __restrict__ row_weight, int64_t A,
+    int splits, int cpb, uint16_t* __restrict__ contrib, GemmCapture cap) {
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kDownTokens + 8 * 4096];
+  const int p = blockIdx.x;
+  const int slot = p >> 3;
+  const int mt = (slot / (2 * splits)) * 8 + (p & 7);
+  if (mt >= *tile_count) return;
+  const int sub = slot % (2 * splits), half = sub / splits;
+  const int tile_rows = tiles[4 * mt + 2];
+  if (half * kDownRows >= tile_rows) return;
+  const int chunks = L.hidden / kDownChunk;
+  const int c0 = (sub % splits) * cpb, c1 = min(chunks, c0 + cpb);
+  DownTile t;
+  t.e = tiles[4 * mt + 0];
+  t.row0 = tiles[4 * mt + 1] + half * kDownRows;
+  t.rows = min(kDownRows, tile_rows - half * kDownRows);
+  t.GK = L.inter >> 7;
+  if (t.rows <= 32) {
+    const ThinArgs a{act, tiles, tile_count, nullptr, row_weight, A, 0,
+                     nullptr, contrib, nullptr, cap.contrib32};
+    for (int nt = c0 / 4; nt < c1 / 4; ++nt) {  // 256 columns each
+      if (nt > c0 / 4) __syncthreads();
+      if (t.rows <= 16) {
+        thin_tile<false, 1, kThinTurn, V4, CAP, 512>(a, L, smem, t.e, t.row0, t.rows, nt);
+      } else {
+        thin_tile<false, 2, kThinTurn, V4, CAP, 512>(a, L, smem, t.e, t.row0, t.rows, nt);
+      }
+    }
+    return;
+  }
+  t.chunk0 = c0 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  t.chunks = c1;
+  switch ((t.rows + 31) >> 5) {
+    case 2: down_tile<2, CAP>(t, L, act, row_weight, smem, contrib, cap.contrib32); break;
+    case 3: down_tile<3, CAP>(t, L, act, row_weight, smem, contrib, cap.contrib32); break;
+    default: down_tile<4, CAP>(t, L, act, row_weight, smem, contrib, cap.contrib32); break;
   }
 }
 
@@ -1076,6 +1307,25 @@ static bool thin_vectors(int64_t K, const aima_u4_tensor* const (&w)[4]) {
   return ok;
 }
 
+// Whether the down GEMM keeps a tile's token rows in LDS
+// (grouped_down_kernel): they fit, and the tiles are tall enough that loading
+// them once pays.  Per call (hidden 2048, inter 512, 256 experts, k = 8),
+// resident against grouped_gemm_kernel: T = 777 (24 assignments per expert)
+// 190 against 186 us, T = 1200 (37) 233 against 240, T = 2048 273 against 292
+// (skewed 226 either way), T = 4096 378 against 390.
+static bool down_rows_resident(const PrefillDims& d) {
+  return d.I <= 128 * kDownMaxGroups && d.A > 32 * (int64_t)d.E;
+}
+
+// Its column chunks per block: 8 (one per wave) until 16 still leave six
+// blocks per CU; then the rows are loaded half as often.  T = 8192: 671 us
+// either way; two layers of T = 16384: 2471 us with 16, 2538 with 8; T = 4096
+// 405 and 378.
+static int down_chunks(const PrefillDims& d) {
+  const int64_t halves = (d.A + d.T + kDownRows - 1) / kDownRows;
+  return halves * (d.H / (2 * 8 * kDownChunk)) >= 6 * 256 ? 16 : 8;
+}
+
 // One grouped GEMM of the layer over the schedule's tiles: 16-row tiles in
 // blocks of 256 threads, 256-row tiles in blocks of 512 (tile_rows_log2).
 template <bool GATEUP>
@@ -1086,29 +1336,37 @@ static int launch_gemm(const aima_moe_layer& L, const uint16_t* src, const Prefi
                                             GATEUP ? &L.shared_gate_up : &L.shared_down,
                                             GATEUP ? &L.up : &L.down,
                                             GATEUP ? &L.shared_up : &L.shared_down};
-  const bool v4 = thin_vectors(K, tensors);
+  // instances: vector loads of scales and zero points, value by value, and the
+  // latter with the f32 copies (a branch at every output of a full tile
+  // costs registers, and their spills wait for the stores before them)
+  const bool capture = cap.act32 || cap.contrib32;
+  const bool v4 = thin_vectors(K, tensors) && !capture;
   const unsigned mtiles = (unsigned)round_up(d.max_tiles, 8);
+  auto pick = [&](auto vec, auto gen, auto full) { return v4 ? vec : capture ? full : gen; };
   if (d.bm_log2 == kMinTileLog2) {
     const int nt = GATEUP ? d.I / 64 : d.H / 128;
     const ThinArgs a{src,   w.tiles,   w.tile_count, w.token_map, w.row_weight, d.A, nt,
                      w.act, w.contrib, cap.act32,    cap.contrib32};
-    const dim3 grid(mtiles * nt), block(kThinThreads);
-    const size_t lds = thin_lds_bytes(1, kThinTurn, K / 128);
-    if (v4) {
-      hipLaunchKernelGGL((grouped_thin_kernel<GATEUP, true>), grid, block, lds, st, L, a);
-    } else {
-      hipLaunchKernelGGL((grouped_thin_kernel<GATEUP, false>), grid, block, lds, st, L, a);
-    }
+    hipLaunchKernelGGL(pick(grouped_thin_kernel<GATEUP, true, false>,
+                            grouped_thin_kernel<GATEUP, false, false>,
+                            grouped_thin_kernel<GATEUP, false, true>),
+                       dim3(mtiles * nt), dim3(kThinThreads),
+                       thin_lds_bytes(1, kThinTurn, K / 128), st, L, a);
+  } else if (!GATEUP && down_rows_resident(d)) {
+    const int chunks = d.H / kDownChunk;
+    const int cpb = down_chunks(d);
+    const int splits = (chunks + cpb - 1) / cpb;
+    hipLaunchKernelGGL(pick(grouped_down_kernel<true, false>, grouped_down_kernel<false, false>,
+                            grouped_down_kernel<false, true>),
+                       dim3(mtiles * 2 * splits), dim3(512), 0, st, L, src, w.tiles, w.tile_count,
+                       w.row_weight, d.A, splits, cpb, w.contrib, cap);
   } else {
     const int nt = GATEUP ? d.I / 128 : d.H / 256;
-    const dim3 grid(mtiles * nt), block(kGemmThreads);
-    if (v4) {
-      hipLaunchKernelGGL((grouped_gemm_kernel<GATEUP, true>), grid, block, 0, st, L, src, w.tiles,
-                         w.tile_count, w.token_map, w.row_weight, d.A, nt, w.act, w.contrib, cap);
-    } else {
-      hipLaunchKernelGGL((grouped_gemm_kernel<GATEUP, false>), grid, block, 0, st, L, src, w.tiles,
-                         w.tile_count, w.token_map, w.row_weight, d.A, nt, w.act, w.contrib, cap);
-    }
+    hipLaunchKernelGGL(pick(grouped_gemm_kernel<GATEUP, true, false>,
+                            grouped_gemm_kernel<GATEUP, false, false>,
+                            grouped_gemm_kernel<GATEUP, false, true>),
+                       dim3(mtiles * nt), dim3(kGemmThreads), 0, st, L, src, w.tiles, w.tile_count,
+                       w.token_map, w.row_weight, d.A, nt, w.act, w.contrib, cap);
   }
   return launch_check(GATEUP ? "grouped gate/up GEMM" : "grouped down GEMM");
 }

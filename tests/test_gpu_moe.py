@@ -303,3 +303,39 @@ def test_prefill_thin_tiles(pkg, dev, H, I, experts, shift):
     torch.cuda.synchronize()
     ref = oracle.moe_ffn_tokens(mw, f16_to_f32(x), ids, w.cpu().numpy(), threads=THREADS)
     assert_parity(f16_to_f32(out), ref, what=f"thin tiles H={H} I={I} E={experts}")
+
+
+@pytest.mark.parametrize("H,I", [(256, 128), (768, 256), (512, 384), (1024, 512)])
+@pytest.mark.parametrize("capture", [False, True])
+def test_prefill_resident_down_rows(pkg, dev, H, I, capture):
+    """The down GEMM that keeps a tile's token rows in LDS (inter <= 512, over
+    32 assignments per expert): remainders around each 32-row block of both
+    128-row halves, thin halves, and column counts that leave waves without a
+    chunk (256, 768) or fill whole blocks.  With the f32 copies requested, the
+    f16 contributions are those values rounded.  Tolerance as the other
+    prefill tests."""
+    counts = [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 256, 289]
+    layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=len(counts), seed=400 + H, device=dev)
+    mw = moe_to_oracle(layer)
+    ids = np.repeat(np.arange(len(counts)), counts).astype(np.int32)
+    ids = np.random.default_rng(H + I).permutation(ids)[:, None].copy()
+    T = len(ids)
+    assert T > 32 * len(counts)
+    x = pkg.synth.activations(T, H, 401, dev)
+    w = torch.rand((T, 1), device=dev) + 0.5
+    d_ids = torch.from_numpy(ids).to(dev)
+    if capture:
+        ws, cap = pkg.Workspace(dev), {}
+        out = pkg.grouped_moe_prefill_routed(layer, x, d_ids, w, expert_used_count=1, ws=ws,
+                                             capture_f32=cap)
+        ref = oracle.moe_routed_tokens(mw, f16_to_f32(x), ids, w.cpu().numpy(), threads=THREADS)
+        got = out.cpu().numpy()
+        rows = pkg.prefill_workspace_views(layer, T, 1, ws, with_shared=False)
+        assert torch.equal(rows["contributions"], cap["contributions_f32"].half())
+        assert torch.equal(rows["swiglu"], cap["swiglu_f32"].half())
+    else:
+        out = pkg.grouped_moe_prefill(layer, x, d_ids, w)
+        ref = oracle.moe_ffn_tokens(mw, f16_to_f32(x), ids, w.cpu().numpy(), threads=THREADS)
+        got = f16_to_f32(out)
+    torch.cuda.synchronize()
+    assert_parity(got, ref, what=f"resident down rows H={H} I={I}")
