@@ -1,6 +1,6 @@
 // Grouped MoE prefill on gfx950.
 //
-// 1. Device schedule (three launches): a stable counting sort of the T*k
+// 1. Device schedule (one to three launches): a stable counting sort of the T*k
 //    (token, rank) assignments by expert.  Rows of one expert are ordered by
 //    assignment index, the order of the reference's host BuildGroupedSchedule
 //    (grouped_s8_u4_prefill_runtime.cpp:231-346), so the schedule is
@@ -160,38 +160,41 @@ __device__ __forceinline__ int32_t topk_id(const int32_t* __restrict__ ids, int3
   return ids[(int64_t)(a / k) * stride + a % k];
 }
 
-// One thread per assignment.  Validates the id (range, duplicate among the
-// earlier ranks of its token), ranks it among the block's assignments of the
-// same expert in assignment order (ballot match inside each wave plus the
-// counts of the earlier waves), and writes the block's per-expert counts.
-// The local rank is parked in inverse_map until the scatter.
-__global__ __launch_bounds__(kSchedBlock) void sched_count_kernel(
-    const int32_t* __restrict__ ids, int stride, int32_t A, int k, int E, int bits, uint32_t* err,
-    int32_t* __restrict__ block_counts, int32_t* __restrict__ local_rank) {
-  __shared__ int cnt[kSchedBlock / 64][kMaxExperts];
-  __shared__ int32_t sid[16 + kSchedBlock];
+// One thread per assignment of block `blk`'s 1024.  Validates the id (range,
+// duplicate among the earlier ranks of its token) and ranks it among the
+// block's assignments of the same expert in assignment order (ballot match
+// inside each wave plus the counts of the earlier waves).  Afterwards
+// sh.cnt[w][e] are the counts by wave.
+struct SchedCount {
+  int cnt[kSchedBlock / 64][kMaxExperts];
+  int32_t sid[16 + kSchedBlock];
+};
+__device__ __forceinline__ void sched_count_block(const int32_t* __restrict__ ids, int stride,
+                                                  int32_t A, int k, int E, int bits, uint32_t* err,
+                                                  int32_t blk, SchedCount& sh, int& expert,
+                                                  int& rank_in_block) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int32_t base = (int32_t)blockIdx.x * kSchedBlock;
+  const int32_t base = blk * kSchedBlock;
   for (int w = 0; w < kSchedBlock / 64; ++w) {
-    for (int e = tid; e < E; e += kSchedBlock) cnt[w][e] = 0;
+    for (int e = tid; e < E; e += kSchedBlock) sh.cnt[w][e] = 0;
   }
   // the block's ids and the 16 before them (earlier ranks of a token that
   // starts in the previous block)
   for (int i = tid; i < 16 + kSchedBlock; i += kSchedBlock) {
     const int32_t a = base - 16 + i;
-    sid[i] = (a >= 0 && a < A) ? topk_id(ids, a, k, stride) : -1;
+    sh.sid[i] = (a >= 0 && a < A) ? topk_id(ids, a, k, stride) : -1;
   }
   __syncthreads();
   const int32_t a = base + tid;
   const bool valid = a < A;
   int e = 0;
   if (valid) {
-    const int raw = sid[16 + tid];
+    const int raw = sh.sid[16 + tid];
     const int rank = a % k;
     uint32_t bad = (raw < 0 || raw >= E) ? AIMA_DEVERR_EXPERT_RANGE : 0u;
 #pragma unroll
     for (int p = 1; p < 16; ++p) {
-      if (p <= rank && sid[16 + tid - p] == raw) bad |= AIMA_DEVERR_EXPERT_DUPLICATE;
+      if (p <= rank && sh.sid[16 + tid - p] == raw) bad |= AIMA_DEVERR_EXPERT_DUPLICATE;
     }
     if (bad) atomicOr(err, bad);
     e = (raw < 0 || raw >= E) ? 0 : raw;
@@ -199,19 +202,34 @@ __global__ __launch_bounds__(kSchedBlock) void sched_count_kernel(
   const uint64_t m = match_mask(e, __ballot(valid), bits);
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   const int wrank = __popcll(m & below);
-  if (valid && wrank == 0) cnt[wave][e] = __popcll(m);
+  if (valid && wrank == 0) sh.cnt[wave][e] = __popcll(m);
   __syncthreads();
+  int r = wrank;
   if (valid) {
-    int r = wrank;
-    for (int w = 0; w < wave; ++w) r += cnt[w][e];
-    local_rank[a] = r;
+    for (int w = 0; w < wave; ++w) r += sh.cnt[w][e];
   }
-  for (int x = tid; x < E; x += kSchedBlock) {
-    int s = 0;
+  expert = e;
+  rank_in_block = r;
+}
+
+__device__ __forceinline__ int sched_block_total(const SchedCount& sh, int e) {
+  int s = 0;
 #pragma unroll
-    for (int w = 0; w < kSchedBlock / 64; ++w) s += cnt[w][x];
-    block_counts[(int64_t)blockIdx.x * E + x] = s;
-  }
+  for (int w = 0; w < kSchedBlock / 64; ++w) s += sh.cnt[w][e];
+  return s;
+}
+
+// Counts per block; the local rank is parked in inverse_map until the scatter.
+__global__ __launch_bounds__(kSchedBlock) void sched_count_kernel(
+    const int32_t* __restrict__ ids, int stride, int32_t A, int k, int E, int bits, uint32_t* err,
+    int32_t* __restrict__ block_counts, int32_t* __restrict__ local_rank) {
+  __shared__ SchedCount sh;
+  int e, r;
+  sched_count_block(ids, stride, A, k, E, bits, err, (int32_t)blockIdx.x, sh, e, r);
+  const int32_t a = (int32_t)blockIdx.x * kSchedBlock + threadIdx.x;
+  if (a < A) local_rank[a] = r;
+  for (int x = threadIdx.x; x < E; x += kSchedBlock)
+    block_counts[(int64_t)blockIdx.x * E + x] = sched_block_total(sh, x);
 }
 
 // Exclusive scans of N values per thread over the 1024 threads of a block
@@ -266,41 +284,16 @@ __device__ __forceinline__ int tiles_in_class(int total, int c, int bm_log2) {
   return (c == kTileClasses ? total >> bm_log2 : 0) + (tile_class(rem, bm_log2) == c ? 1 : 0);
 }
 
-// One block of 1024 threads: thread (p, e) with e = tid % Ep (Ep = E rounded
-// up to a power of two) scans chunk p of expert e's block counts, the chunk
-// partial sums are combined through LDS, and the experts' totals are scanned
-// into row offsets and into tile positions per class (class 8 first).
-__global__ __launch_bounds__(1024) void sched_scan_kernel(int32_t* __restrict__ block_base,
-                                                          int32_t nb, int E, int Ep, int32_t T,
-                                                          int32_t A, int with_shared, int bm_log2,
-                                                          int32_t* __restrict__ offsets,
-                                                          int32_t* __restrict__ tiles,
-                                                          int32_t* __restrict__ tile_count) {
-  __shared__ int smem[17 * (1 + kTileClasses)];
-  __shared__ int part[1024];
+// Row offsets and tiles from the experts' totals: the threads with `rep` hold
+// expert e's total.  Every thread gets the exclusive row offset of the
+// experts before its own; offsets, tiles and the tile count are written.
+// `smem` holds 17 * (1 + kTileClasses) ints.
+__device__ __forceinline__ int sched_place_tiles(int total, int e, bool rep, int E, int32_t T,
+                                                 int32_t A, int with_shared, int bm_log2,
+                                                 int32_t* __restrict__ offsets,
+                                                 int32_t* __restrict__ tiles,
+                                                 int32_t* __restrict__ tile_count, int* smem) {
   const int tid = threadIdx.x;
-  const int e = tid % Ep, pidx = tid / Ep, P = 1024 / Ep;
-  const int chunk = (nb + P - 1) / P;
-  const int b0 = pidx * chunk, b1 = min(nb, b0 + chunk);
-  int sum = 0;
-  if (e < E) {
-    for (int b = b0; b < b1; b += 16) {
-      int c[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) c[j] = b + j < b1 ? block_base[(int64_t)(b + j) * E + e] : 0;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) sum += c[j];
-    }
-  }
-  part[tid] = sum;
-  __syncthreads();
-  int before = 0, total = 0;
-  for (int q = 0; q < P; ++q) {
-    const int v = part[q * Ep + e];
-    if (q < pidx) before += v;
-    total += v;
-  }
-  const bool rep = pidx == 0 && e < E;
   // one scan for the row offsets and the tile counts of every class
   // (v[0] rows, v[c] tiles of class c)
   int v[1 + kTileClasses], tot[1 + kTileClasses];
@@ -310,22 +303,6 @@ __global__ __launch_bounds__(1024) void sched_scan_kernel(int32_t* __restrict__ 
   block_exclusive_scan_1024<1 + kTileClasses>(v, tot, smem);
   const int begin = v[0];
   if (rep) offsets[e] = begin + total;
-  // expert e's row base reaches every chunk thread through LDS
-  if (pidx == 0) part[e] = begin;
-  __syncthreads();
-  if (e < E) {
-    int run = part[e] + before;
-    for (int b = b0; b < b1; b += 16) {
-      int c[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) c[j] = b + j < b1 ? block_base[(int64_t)(b + j) * E + e] : 0;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        if (b + j < b1) block_base[(int64_t)(b + j) * E + e] = run;
-        run += c[j];
-      }
-    }
-  }
   // Tiles, by class (tallest first); the shared expert's tiles follow the
   // routed ones of each class.  An expert has full tiles (class 8) and at
   // most one remainder tile.
@@ -369,6 +346,63 @@ __global__ __launch_bounds__(1024) void sched_scan_kernel(int32_t* __restrict__ 
     if (with_shared) place(E, A, T, cbase[kTileClasses] + tot[kTileClasses], rem_slot(T, tot));
     *tile_count = all_tiles;
   }
+  return begin;
+}
+
+// One block of 1024 threads: thread (p, e) with e = tid % Ep (Ep = E rounded
+// up to a power of two) scans chunk p of expert e's block counts, the chunk
+// partial sums are combined through LDS, and the experts' totals are scanned
+// into row offsets and into tile positions per class (class 8 first).  For
+// schedules of more blocks than sched_rows_kernel takes.
+__global__ __launch_bounds__(1024) void sched_scan_kernel(int32_t* __restrict__ block_base,
+                                                          int32_t nb, int E, int Ep, int32_t T,
+                                                          int32_t A, int with_shared, int bm_log2,
+                                                          int32_t* __restrict__ offsets,
+                                                          int32_t* __restrict__ tiles,
+                                                          int32_t* __restrict__ tile_count) {
+  __shared__ int smem[17 * (1 + kTileClasses)];
+  __shared__ int part[1024];
+  const int tid = threadIdx.x;
+  const int e = tid % Ep, pidx = tid / Ep, P = 1024 / Ep;
+  const int chunk = (nb + P - 1) / P;
+  const int b0 = pidx * chunk, b1 = min(nb, b0 + chunk);
+  int sum = 0;
+  if (e < E) {
+    for (int b = b0; b < b1; b += 16) {
+      int c[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) c[j] = b + j < b1 ? block_base[(int64_t)(b + j) * E + e] : 0;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) sum += c[j];
+    }
+  }
+  part[tid] = sum;
+  __syncthreads();
+  int before = 0, total = 0;
+  for (int q = 0; q < P; ++q) {
+    const int v = part[q * Ep + e];
+    if (q < pidx) before += v;
+    total += v;
+  }
+  const bool rep = pidx == 0 && e < E;
+  const int begin = sched_place_tiles(total, e, rep, E, T, A, with_shared, bm_log2, offsets, tiles,
+                                      tile_count, smem);
+  // expert e's row base reaches every chunk thread through LDS
+  if (pidx == 0) part[e] = begin;
+  __syncthreads();
+  if (e < E) {
+    int run = part[e] + before;
+    for (int b = b0; b < b1; b += 16) {
+      int c[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) c[j] = b + j < b1 ? block_base[(int64_t)(b + j) * E + e] : 0;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        if (b + j < b1) block_base[(int64_t)(b + j) * E + e] = run;
+        run += c[j];
+      }
+    }
+  }
 }
 
 // One thread per assignment: the row = block base of its expert + its local
@@ -385,6 +419,89 @@ __global__ __launch_bounds__(kSchedBlock) void sched_scatter_kernel(
   token_map[pos] = a / k;
   inverse_map[a] = pos;
   row_weight[pos] = weights[a];
+}
+
+// The rest of a schedule in one launch.  Every block sums the counts of all
+// blocks and of the blocks before it (thread (p, e) chunk p of expert e's, as
+// in sched_scan_kernel), scans the experts' totals into its row bases and
+// places its own 1024 assignments; block 0 also writes offsets and tiles.
+// With ONE (a single block) the counts are its own, and the whole schedule is
+// this launch.  Latency-bound (7 to 14 us): what it saves is launches, T = 7
+// 39.0 -> 35.1 us per call, T = 96 105.2 -> 100.4, two layers of T = 16384
+// (128 blocks) 2423 -> 2416.  The counts are read by every block (E * 4 bytes
+// each), so past kSchedRowsBlocks blocks the scan stays a launch of its own.
+constexpr int kSchedRowsBlocks = 256;
+
+template <bool ONE>
+__global__ __launch_bounds__(kSchedBlock) void sched_rows_kernel(
+    const int32_t* __restrict__ ids, int stride, const float* __restrict__ weights, int32_t A,
+    int k, int E, int Ep, int bits, uint32_t* err, const int32_t* __restrict__ block_counts,
+    int32_t T, int with_shared, int bm_log2, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count, int32_t* __restrict__ token_map,
+    int32_t* __restrict__ inverse_map, float* __restrict__ row_weight) {
+  __shared__ int smem[17 * (1 + kTileClasses)];
+  __shared__ int part[1024], part_before[1024];
+  __shared__ int base[kMaxExperts];
+  const int tid = threadIdx.x;
+  const int32_t blk = blockIdx.x, nb = gridDim.x;
+  const int32_t a = blk * kSchedBlock + tid;
+  int my_e = 0, my_rank = 0;
+  float wt = 0.f;
+  if (a < A) wt = weights[a];
+  const int e = tid % Ep, pidx = tid / Ep, P = 1024 / Ep;
+  int total = 0, before = 0;
+  if constexpr (ONE) {
+    __shared__ SchedCount sh;
+    sched_count_block(ids, stride, A, k, E, bits, err, 0, sh, my_e, my_rank);
+    if (e < E) total = sched_block_total(sh, e);
+  } else {
+    if (a < A) {
+      const int raw = topk_id(ids, a, k, stride);
+      my_e = (raw < 0 || raw >= E) ? 0 : raw;
+      my_rank = inverse_map[a];
+    }
+    const int chunk = (nb + P - 1) / P;
+    const int b0 = pidx * chunk, b1 = min(nb, b0 + chunk);
+    int sum = 0, early = 0;
+    if (e < E) {
+      for (int b = b0; b < b1; b += 16) {
+        int c[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          c[j] = b + j < b1 ? block_counts[(int64_t)(b + j) * E + e] : 0;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          sum += c[j];
+          early += b + j < blk ? c[j] : 0;
+        }
+      }
+    }
+    part[tid] = sum;
+    part_before[tid] = early;
+    __syncthreads();
+    for (int q = 0; q < P; ++q) {
+      total += part[q * Ep + e];
+      before += part_before[q * Ep + e];
+    }
+  }
+  const bool rep = pidx == 0 && e < E;
+  int begin;
+  if (blk == 0) {
+    begin = sched_place_tiles(total, e, rep, E, T, A, with_shared, bm_log2, offsets, tiles,
+                              tile_count, smem);
+  } else {
+    int v[1] = {rep ? total : 0}, tot[1];
+    block_exclusive_scan_1024<1>(v, tot, smem);
+    begin = v[0];
+  }
+  if (rep) base[e] = begin + before;
+  __syncthreads();
+  if (a < A) {
+    const int pos = base[my_e] + my_rank;
+    token_map[pos] = a / k;
+    inverse_map[a] = pos;
+    row_weight[pos] = wt;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1271,13 +1388,28 @@ static int launch_schedule(const int32_t* ids, int stride, const float* weights,
   const int bits = expert_bits(d.E);
   int Ep = 1;
   while (Ep < d.E) Ep <<= 1;
+  const int shared = with_shared ? 1 : 0;
+  if (d.nb == 1) {
+    hipLaunchKernelGGL(sched_rows_kernel<true>, dim3(1), dim3(kSchedBlock), 0, st, ids, stride,
+                       weights, (int32_t)d.A, d.k, d.E, Ep, bits, w.err, w.block_base, (int32_t)d.T,
+                       shared, d.bm_log2, w.offsets, w.tiles, w.tile_count, w.token_map,
+                       w.inverse_map, w.row_weight);
+    return launch_check("grouped schedule");
+  }
   hipLaunchKernelGGL(sched_count_kernel, dim3((unsigned)d.nb), dim3(kSchedBlock), 0, st, ids,
                      stride, (int32_t)d.A, d.k, d.E, bits, w.err, w.block_base, w.inverse_map);
   int rc = launch_check("grouped schedule count");
   if (rc != AIMA_OK) return rc;
+  if (d.nb <= kSchedRowsBlocks) {
+    hipLaunchKernelGGL(sched_rows_kernel<false>, dim3((unsigned)d.nb), dim3(kSchedBlock), 0, st,
+                       ids, stride, weights, (int32_t)d.A, d.k, d.E, Ep, bits, w.err, w.block_base,
+                       (int32_t)d.T, shared, d.bm_log2, w.offsets, w.tiles, w.tile_count,
+                       w.token_map, w.inverse_map, w.row_weight);
+    return launch_check("grouped schedule rows");
+  }
   hipLaunchKernelGGL(sched_scan_kernel, dim3(1), dim3(1024), 0, st, w.block_base, (int32_t)d.nb,
-                     d.E, Ep, (int32_t)d.T, (int32_t)d.A, with_shared ? 1 : 0, d.bm_log2, w.offsets,
-                     w.tiles, w.tile_count);
+                     d.E, Ep, (int32_t)d.T, (int32_t)d.A, shared, d.bm_log2, w.offsets, w.tiles,
+                     w.tile_count);
   rc = launch_check("grouped schedule scan");
   if (rc != AIMA_OK) return rc;
   hipLaunchKernelGGL(sched_scatter_kernel, dim3((unsigned)d.nb), dim3(kSchedBlock), 0, st, ids,

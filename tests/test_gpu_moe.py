@@ -339,3 +339,17 @@ def test_prefill_resident_down_rows(pkg, dev, H, I, capture):
         got = f16_to_f32(out)
     torch.cuda.synchronize()
     assert_parity(got, ref, what=f"resident down rows H={H} I={I}")
+
+
+@pytest.mark.parametrize("T,E,k", [(128, 256, 8), (1025, 8, 1), (147, 1024, 7), (32768, 256, 8),
+                                   (32770, 130, 8)])
+def test_schedule_launch_forms(pkg, dev, T, E, k):
+    """A schedule of one block of assignments (1024, one launch), just past
+    it, and around the most blocks whose row bases every block sums itself
+    (256; beyond, the scan is a launch of its own).  Integers: exact."""
+    ids, w = pkg.select_router_topk(pkg.synth.router_logits(T, E, seed=T + E, device=dev), k)
+    s = pkg.build_grouped_schedule(ids, w, E)
+    torch.cuda.synchronize()
+    r = oracle.build_grouped_schedule(ids.cpu().numpy(), E, w.cpu().numpy())
+    for name in ("offsets", "token_map", "inverse_map", "compact_weights"):
+        assert np.array_equal(s[name].cpu().numpy(), r[name]), name
