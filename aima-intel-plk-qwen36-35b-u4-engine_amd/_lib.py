@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 import torch  # noqa: F401  (loads the HIP runtime before the library)
 
@@ -68,6 +69,34 @@ class FfnTraceC(C.Structure):
         "selected_gate_up", "selected_swiglu", "selected_down", "weighted_selected_down",
         "moe_out", "shared_gate", "shared_gate_sigmoid", "shared_gate_up", "shared_swiglu",
         "shared_down", "shared_gated", "ffn_out", "residual")]
+
+
+def u4_tensors(weights):
+    """Array of U4TensorC over U4 weights.  Filled from packed addresses: a
+    ctypes structure per tensor costs about a microsecond of host time."""
+    flat = []
+    for w in weights:
+        flat += (w.qweight.data_ptr(), w.scale.data_ptr(), w.zp.data_ptr())
+    return (U4TensorC * len(weights)).from_buffer_copy(struct.pack(f"{len(flat)}Q", *flat))
+
+
+# MoeLayerC as struct.pack lays it out: four tensors and two vectors, five
+# sizes (padded to the next pointer), two tensors
+_MOE_LAYER = struct.Struct("14Q5i4x6Q")
+assert _MOE_LAYER.size == C.sizeof(MoeLayerC)
+
+
+def moe_layer_c(gate_up, down, shared_gate_up, shared_down, gate_vec, norm, sizes, up, shared_up):
+    """MoeLayerC from U4 weights (up, shared_up may be None), addresses and the
+    sizes (hidden, inter, shared_inter, experts, group)."""
+    flat = []
+    for w in (gate_up, down, shared_gate_up, shared_down):
+        flat += (w.qweight.data_ptr(), w.scale.data_ptr(), w.zp.data_ptr())
+    tail = []
+    for w in (up, shared_up):
+        tail += (0, 0, 0) if w is None else (w.qweight.data_ptr(), w.scale.data_ptr(),
+                                             w.zp.data_ptr())
+    return MoeLayerC.from_buffer_copy(_MOE_LAYER.pack(*flat, gate_vec, norm, *sizes, *tail))
 
 
 _LP = C.POINTER(MoeLayerC)

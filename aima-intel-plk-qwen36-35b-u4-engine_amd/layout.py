@@ -19,7 +19,7 @@ from typing import Optional
 
 import torch
 
-from ._lib import MoeLayerC, U4TensorC
+from ._lib import MoeLayerC, U4TensorC, moe_layer_c
 
 
 @dataclass
@@ -152,13 +152,11 @@ class MoeLayerWeights:
         return self.shared_gate_up.nbytes + up + self.shared_down.nbytes
 
     def c(self) -> MoeLayerC:
-        none = U4TensorC(None, None, None)
-        return MoeLayerC(self.gate_up.c(), self.down.c(), self.shared_gate_up.c(),
-                         self.shared_down.c(), self.shared_gate_vec.data_ptr(),
-                         self.norm_weight.data_ptr() if self.norm_weight is not None else None,
-                         self.hidden, self.inter, self.shared_inter, self.experts, self.group,
-                         self.up.c() if self.split else none,
-                         self.shared_up.c() if self.split else none)
+        return moe_layer_c(self.gate_up, self.down, self.shared_gate_up, self.shared_down,
+                           self.shared_gate_vec.data_ptr(),
+                           self.norm_weight.data_ptr() if self.norm_weight is not None else 0,
+                           (self.hidden, self.inter, self.shared_inter, self.experts, self.group),
+                           self.up, self.shared_up if self.split else None)
 
     def to_split(self) -> "MoeLayerWeights":
         """The same layer in the split form (copies of the gate and up rows)."""
