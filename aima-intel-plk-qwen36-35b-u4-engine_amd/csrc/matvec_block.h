@@ -65,6 +65,85 @@ __device__ __forceinline__ void build_x_chunks(const u32x4 (&xr)[RowGeom<KCH>::N
   }
 }
 
+// Where a block's activations come from: issue() starts their loads (before
+// the weights'), finish() hands over the lane's chunks.
+template <int KCH>
+struct XGlobal {
+  const uint16_t* __restrict__ x;
+  u32x4 xr[RowGeom<KCH>::NC][4];
+  __device__ __forceinline__ void issue(int cl) { load_x_raw<KCH>(x, cl, xr); }
+  __device__ __forceinline__ void finish(int, u32x4 (&out)[RowGeom<KCH>::NC][4]) {
+#pragma unroll
+    for (int i = 0; i < RowGeom<KCH>::NC; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) out[i][q] = xr[i][q];
+  }
+};
+
+// The RMSNorm of a row, formed by every block for itself while its weights
+// are in flight (rmsnorm_row's arithmetic and summation order: the same bits);
+// `store`: this block also writes it to h.
+template <int KCH>
+struct XNorm {
+  static constexpr int K = RowGeom<KCH>::K;
+  static constexpr int kChunks = (K / 8 + 255) / 256;  // 8-element chunks per thread
+  const uint16_t* __restrict__ r;
+  const float* __restrict__ weight;
+  float eps;
+  uint16_t* __restrict__ h;
+  bool store;
+  uint16_t* lds;  // [K]
+  float* red;     // [4]
+  u32x4 v[kChunks];
+  float w[kChunks][8];
+  __device__ __forceinline__ void issue(int) {
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const int i = (threadIdx.x + 256 * c) * 8, ic = i < K ? i : 0;
+      v[c] = *reinterpret_cast<const u32x4*>(r + ic);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[c][j] = weight[ic + j];
+    }
+  }
+  __device__ __forceinline__ void finish(int cl, u32x4 (&out)[RowGeom<KCH>::NC][4]) {
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      if ((int)(threadIdx.x + 256 * c) * 8 < K) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float lo = h2f((uint16_t)(v[c][j] & 0xffffu)), hi = h2f((uint16_t)(v[c][j] >> 16));
+          ss = fmaf(lo, lo, ss);
+          ss = fmaf(hi, hi, ss);
+        }
+      }
+    }
+    ss = block_sum_256(ss, red);
+    const float scale = 1.0f / sqrtf(ss / (float)(int64_t)K + eps);
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const int i = (threadIdx.x + 256 * c) * 8;
+      if (i < K) {
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float lo = h2f((uint16_t)(v[c][j] & 0xffffu)) * scale * w[c][2 * j];
+          const float hi = h2f((uint16_t)(v[c][j] >> 16)) * scale * w[c][2 * j + 1];
+          o[j] = pack_h2(lo, hi);
+        }
+        *reinterpret_cast<u32x4*>(lds + i) = o;
+        if (store) *reinterpret_cast<u32x4*>(h + i) = o;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RowGeom<KCH>::NC; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        out[i][q] = *reinterpret_cast<const u32x4*>(lds + (cl + i * RowGeom<KCH>::SEG) * 32 + 8 * q);
+  }
+};
+
 // Rows blk * BR .. +BR of one matrix (the body of every matvec block).
 //
 // Load order: the block's scales and zero points (contiguous: its rows are
@@ -76,9 +155,9 @@ __device__ __forceinline__ void build_x_chunks(const u32x4 (&xr)[RowGeom<KCH>::N
 // tagged (optional; used only where a wave pass covers one row, K >= 2048):
 // the f32 result of row r is also stored as the 64-bit word {bits, logit_tag(bits, tag)} at
 // tagged[r] (the LM head's fused top-k reads those).
-template <int KCH, int RG>
+template <int KCH, int RG, class XSource>
 __device__ __forceinline__ void matvec_block(
-    const uint16_t* __restrict__ x, const uint8_t* __restrict__ qw,
+    XSource& xs, const uint8_t* __restrict__ qw,
     const uint16_t* __restrict__ scale, const uint8_t* __restrict__ zp,
     int64_t n, int group_log2, void* __restrict__ y, int out_f32, int64_t blk,
     uint64_t* __restrict__ tagged = nullptr, uint32_t tag = 0) {
@@ -121,8 +200,7 @@ __device__ __forceinline__ void matvec_block(
     const int i = tid + 256 * j;
     zw[j] = i < z_full ? reinterpret_cast<const uint32_t*>(zblk)[i] : 0u;
   }
-  u32x4 xr[G::NC][4];
-  load_x_raw<KCH>(x, cl, xr);
+  xs.issue(cl);
   // rows past n load row n - 1 instead (straight-line loads, no branch
   // around each); their results are never written
   u32x4 w[RG][G::NC];
@@ -148,6 +226,8 @@ __device__ __forceinline__ void matvec_block(
   }
   for (int t = 2 * s_full + tid; t < nsc; t += 256) s_lds[t] = sblk[t];
   for (int t = 4 * z_full + tid; t < zbytes; t += 256) z_lds[t] = zblk[t];
+  u32x4 xr[G::NC][4];
+  xs.finish(cl, xr);
   XChunk xc[G::NC];
   build_x_chunks<KCH>(xr, xc);
   __syncthreads();
@@ -195,6 +275,17 @@ __device__ __forceinline__ void matvec_block(
       }
     }
   }
+}
+
+template <int KCH, int RG>
+__device__ __forceinline__ void matvec_block(
+    const uint16_t* __restrict__ x, const uint8_t* __restrict__ qw,
+    const uint16_t* __restrict__ scale, const uint8_t* __restrict__ zp,
+    int64_t n, int group_log2, void* __restrict__ y, int out_f32, int64_t blk,
+    uint64_t* __restrict__ tagged = nullptr, uint32_t tag = 0) {
+  XGlobal<KCH> xs;
+  xs.x = x;
+  matvec_block<KCH, RG>(xs, qw, scale, zp, n, group_log2, y, out_f32, blk, tagged, tag);
 }
 
 }  // namespace aima

@@ -14,6 +14,7 @@
 // w_s * (row . act_s) over its slots, and the eight partial sums plus the
 // residual are added in a fixed order: no atomics, deterministic.
 #include "common.h"
+#include "matvec_block.h"
 
 #include <math.h>
 
@@ -806,6 +807,53 @@ static int check_routed_stack(const aima_moe_layer* layers, const aima_u4_tensor
 }
 
 // The routed stack decode's launches on workspace w (its error word is w.err).
+namespace {
+
+// Layer input and router of the routed stack in one launch: logits = router .
+// h with h = rmsnorm(r), formed by every block beside its router rows' loads
+// and written to h by block 0 (the same bits as rmsnorm_launch and the matvec).
+// Against the two launches (and the slower selection before it), four layers
+// of hidden 1024, 64 experts: 65.3 -> 55.4 us a token.
+template <int KCH>
+__global__ __launch_bounds__(256) void norm_router_kernel(
+    const uint16_t* __restrict__ r, const float* __restrict__ norm, float eps,
+    aima_u4_tensor router, int experts, int group_log2, uint16_t* __restrict__ h,
+    float* __restrict__ logits) {
+  __shared__ __attribute__((aligned(16))) uint16_t lds[RowGeom<KCH>::K];
+  __shared__ float red[4];
+  XNorm<KCH> xs;
+  xs.r = r;
+  xs.weight = norm;
+  xs.eps = eps;
+  xs.h = h;
+  xs.store = blockIdx.x == 0;
+  xs.lds = lds;
+  xs.red = red;
+  matvec_block<KCH, 4>(xs, router.qweight, router.scale, router.zp, (int64_t)experts, group_log2,
+                       logits, 1, (int64_t)blockIdx.x);
+}
+
+static int norm_router_launch(const uint16_t* r, const aima_moe_layer& L, float eps,
+                              const aima_u4_tensor& router, uint16_t* h, float* logits,
+                              hipStream_t st) {
+  AIMA_REQUIRE(aligned(r, 16), "moe stack: the residual must be 16-byte aligned");
+  auto launch = [&](auto kernel, int rows_per_pass) {
+    const int br = 16 * rows_per_pass;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((L.experts + br - 1) / br)), dim3(256), 0, st, r,
+                       L.norm_weight, eps, router, L.experts, group_log2_of(L.group), h, logits);
+  };
+  switch (L.hidden / 32) {
+    case 16: launch(norm_router_kernel<16>, RowGeom<16>::RPI); break;
+    case 32: launch(norm_router_kernel<32>, RowGeom<32>::RPI); break;
+    case 64: launch(norm_router_kernel<64>, RowGeom<64>::RPI); break;
+    case 128: launch(norm_router_kernel<128>, RowGeom<128>::RPI); break;
+    default: return fail(AIMA_E_UNSUPPORTED, "moe stack: unsupported hidden size");
+  }
+  return launch_check("moe stack norm and router");
+}
+
+}  // namespace
+
 static int routed_stack_run(const aima_moe_layer* layers, const aima_u4_tensor* routers,
                             int32_t n_layers, float eps, const uint16_t* residual_in, int32_t k,
                             float min_weight_sum, int32_t* ids, float* weights, uint16_t* out,
@@ -813,11 +861,8 @@ static int routed_stack_run(const aima_moe_layer* layers, const aima_u4_tensor* 
   const uint16_t* r = residual_in;
   for (int32_t l = 0; l < n_layers; ++l) {
     const aima_moe_layer& L = layers[l];
-    int rc = rmsnorm_launch(r, L.norm_weight, 1, L.hidden, eps, w.h, st);
-    if (rc != AIMA_OK) return rc;
     // routing from this layer's normalized input (gguf_loader.cpp:5708-5711)
-    rc = u4_matvec_dispatch(w.h, routers[l].qweight, routers[l].scale, routers[l].zp, L.experts,
-                            L.hidden, group_log2_of(L.group), w.logits, 1, st);
+    int rc = norm_router_launch(r, L, eps, routers[l], w.h, w.logits, st);
     if (rc != AIMA_OK) return rc;
     int32_t* ids_l = ids + (int64_t)l * k;
     float* w_l = weights + (int64_t)l * k;

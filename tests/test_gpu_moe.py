@@ -353,3 +353,19 @@ def test_schedule_launch_forms(pkg, dev, T, E, k):
     r = oracle.build_grouped_schedule(ids.cpu().numpy(), E, w.cpu().numpy())
     for name in ("offsets", "token_map", "inverse_map", "compact_weights"):
         assert np.array_equal(s[name].cpu().numpy(), r[name]), name
+
+
+@pytest.mark.parametrize("E,k", [(5, 5), (64, 16), (65, 3), (256, 8), (256, 16), (1000, 16)])
+def test_router_selection_ties(pkg, dev, E, k):
+    """Equal probabilities across lanes, within a lane (ids 64 apart) and
+    everywhere, and fewer finite logits than picks: ids exact, lowest first."""
+    g = np.random.default_rng(E + k)
+    rows = [np.zeros(E), np.round(g.normal(size=E)), g.normal(size=E),
+            np.tile(g.normal(size=64), -(-E // 64))[:E], np.full(E, -np.inf)]
+    rows[4][g.permutation(E)[:max(1, k // 2)]] = 1.0
+    logits = np.stack(rows).astype(np.float32)
+    ids, w = pkg.select_router_topk(torch.from_numpy(logits).to(dev), k)
+    torch.cuda.synchronize()
+    ref_ids, ref_w = oracle.router_topk_tokens(logits, k)
+    assert np.array_equal(ids.cpu().numpy(), ref_ids)
+    assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")

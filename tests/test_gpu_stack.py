@@ -479,3 +479,23 @@ def test_stack_decode_routed_true_decode(pkg, dev):
         o2 = oracle.moe_ffn_tokens(lnp[l], h, rid, rw, residual=rf, threads=THREADS)
         r = oracle.float_to_half(o2).reshape(o2.shape)
     assert checked >= 2
+
+
+@pytest.mark.parametrize("H,I,E,group,k", [(512, 128, 17, 64, 1), (1024, 256, 33, 32, 4),
+                                           (2048, 512, 300, 128, 8), (4096, 128, 16, 256, 16)])
+def test_routed_stack_equals_single_calls(pkg, dev, H, I, E, group, k):
+    """The routed stack's fused norm and router (every hidden size, partial
+    router blocks, all groups) gives the bits of the separate calls."""
+    layers = [pkg.synth.moe_layer(hidden=H, inter=I if I % group == 0 else 256, experts=E,
+                                  group=group, seed=500 + H + l, device=dev) for l in range(2)]
+    routers = [pkg.synth.u4_weight(1, E, H, group, pkg.synth.generator(600 + l, dev), dev)
+               for l in range(2)]
+    x = pkg.synth.activations(1, H, 501, dev)[0].contiguous()
+    out, ids, w = pkg.moe_stack_decode_routed(layers, routers, x, k)
+    r = x
+    for l in range(2):
+        h = pkg.apply_rms_norm(r, layers[l].norm_weight, 1e-6)
+        i1, w1, _ = pkg.router_fc_topk(h, routers[l], k)
+        r = pkg.run_moe_ffn_layer(layers[l], h, i1, w1, residual=r)
+        assert torch.equal(ids[l], i1) and torch.equal(w[l], w1), l
+    assert torch.equal(out, r)
