@@ -219,11 +219,35 @@ __device__ __forceinline__ int sched_block_total(const SchedCount& sh, int e) {
   return s;
 }
 
+// f32 hidden states (RunLayer's input type) -> f16 GEMM operands, round to
+// nearest even, 8 values per thread: done by blocks of the schedule's first
+// launch that have no assignments (a launch of its own took 5 us at T = 777).
+struct InputF32 {
+  const float4* in;  // null: the input is f16
+  u32x4* out;
+  int64_t n8;
+};
+__device__ __forceinline__ void convert_f32_block(const InputF32& x, int64_t blk) {
+  const int64_t i = blk * kSchedBlock + threadIdx.x;
+  if (i >= x.n8) return;
+  const float4 a = x.in[2 * i], b = x.in[2 * i + 1];
+  x.out[i] = u32x4{pack_h2(a.x, a.y), pack_h2(a.z, a.w), pack_h2(b.x, b.y), pack_h2(b.z, b.w)};
+}
+static unsigned convert_blocks(const InputF32& x) {
+  return x.in ? (unsigned)((x.n8 + kSchedBlock - 1) / kSchedBlock) : 0u;
+}
+
 // Counts per block; the local rank is parked in inverse_map until the scatter.
+// Blocks from nb on convert an f32 input.
 __global__ __launch_bounds__(kSchedBlock) void sched_count_kernel(
     const int32_t* __restrict__ ids, int stride, int32_t A, int k, int E, int bits, uint32_t* err,
-    int32_t* __restrict__ block_counts, int32_t* __restrict__ local_rank) {
+    int32_t nb, int32_t* __restrict__ block_counts, int32_t* __restrict__ local_rank,
+    InputF32 input) {
   __shared__ SchedCount sh;
+  if ((int32_t)blockIdx.x >= nb) {
+    convert_f32_block(input, (int64_t)blockIdx.x - nb);
+    return;
+  }
   int e, r;
   sched_count_block(ids, stride, A, k, E, bits, err, (int32_t)blockIdx.x, sh, e, r);
   const int32_t a = (int32_t)blockIdx.x * kSchedBlock + threadIdx.x;
@@ -426,7 +450,7 @@ __global__ __launch_bounds__(kSchedBlock) void sched_scatter_kernel(
 // in sched_scan_kernel), scans the experts' totals into its row bases and
 // places its own 1024 assignments; block 0 also writes offsets and tiles.
 // With ONE (a single block) the counts are its own, and the whole schedule is
-// this launch.  Latency-bound (7 to 14 us): what it saves is launches, T = 7
+// this launch (further blocks convert an f32 input).  Latency-bound (7 to 14 us): what it saves is launches, T = 7
 // 39.0 -> 35.1 us per call, T = 96 105.2 -> 100.4, two layers of T = 16384
 // (128 blocks) 2423 -> 2416.  The counts are read by every block (E * 4 bytes
 // each), so past kSchedRowsBlocks blocks the scan stays a launch of its own.
@@ -438,12 +462,16 @@ __global__ __launch_bounds__(kSchedBlock) void sched_rows_kernel(
     int k, int E, int Ep, int bits, uint32_t* err, const int32_t* __restrict__ block_counts,
     int32_t T, int with_shared, int bm_log2, int32_t* __restrict__ offsets,
     int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count, int32_t* __restrict__ token_map,
-    int32_t* __restrict__ inverse_map, float* __restrict__ row_weight) {
+    int32_t* __restrict__ inverse_map, float* __restrict__ row_weight, InputF32 input) {
   __shared__ int smem[17 * (1 + kTileClasses)];
   __shared__ int part[1024], part_before[1024];
   __shared__ int base[kMaxExperts];
   const int tid = threadIdx.x;
-  const int32_t blk = blockIdx.x, nb = gridDim.x;
+  const int32_t blk = blockIdx.x, nb = gridDim.x;  // (nb is not used with ONE)
+  if (ONE && blk > 0) {
+    convert_f32_block(input, (int64_t)blk - 1);
+    return;
+  }
   const int32_t a = blk * kSchedBlock + tid;
   int my_e = 0, my_rank = 0;
   float wt = 0.f;
@@ -1361,16 +1389,6 @@ __global__ __launch_bounds__(256) void combine_routed_f32_kernel(
   }
 }
 
-// f32 hidden states (RunLayer's input type) -> f16 GEMM operands, round to
-// nearest even; 8 values per thread.
-__global__ __launch_bounds__(256) void f32_to_f16_kernel(const float4* __restrict__ in,
-                                                         int64_t n8, u32x4* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n8) return;
-  const float4 a = in[2 * i], b = in[2 * i + 1];
-  out[i] = u32x4{pack_h2(a.x, a.y), pack_h2(a.z, a.w), pack_h2(b.x, b.y), pack_h2(b.z, b.w)};
-}
-
 // ---------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------
@@ -1384,27 +1402,29 @@ static int expert_bits(int E) {
 // shared expert's tiles (rows A .. A + T - 1).
 static int launch_schedule(const int32_t* ids, int stride, const float* weights,
                            const PrefillDims& d, const PrefillWs& w, bool with_shared,
-                           hipStream_t st) {
+                           const InputF32& input, hipStream_t st) {
   const int bits = expert_bits(d.E);
   int Ep = 1;
   while (Ep < d.E) Ep <<= 1;
   const int shared = with_shared ? 1 : 0;
+  const unsigned conv = convert_blocks(input);
   if (d.nb == 1) {
-    hipLaunchKernelGGL(sched_rows_kernel<true>, dim3(1), dim3(kSchedBlock), 0, st, ids, stride,
+    hipLaunchKernelGGL(sched_rows_kernel<true>, dim3(1 + conv), dim3(kSchedBlock), 0, st, ids, stride,
                        weights, (int32_t)d.A, d.k, d.E, Ep, bits, w.err, w.block_base, (int32_t)d.T,
                        shared, d.bm_log2, w.offsets, w.tiles, w.tile_count, w.token_map,
-                       w.inverse_map, w.row_weight);
+                       w.inverse_map, w.row_weight, input);
     return launch_check("grouped schedule");
   }
-  hipLaunchKernelGGL(sched_count_kernel, dim3((unsigned)d.nb), dim3(kSchedBlock), 0, st, ids,
-                     stride, (int32_t)d.A, d.k, d.E, bits, w.err, w.block_base, w.inverse_map);
+  hipLaunchKernelGGL(sched_count_kernel, dim3((unsigned)d.nb + conv), dim3(kSchedBlock), 0, st, ids,
+                     stride, (int32_t)d.A, d.k, d.E, bits, w.err, (int32_t)d.nb, w.block_base,
+                     w.inverse_map, input);
   int rc = launch_check("grouped schedule count");
   if (rc != AIMA_OK) return rc;
   if (d.nb <= kSchedRowsBlocks) {
     hipLaunchKernelGGL(sched_rows_kernel<false>, dim3((unsigned)d.nb), dim3(kSchedBlock), 0, st,
                        ids, stride, weights, (int32_t)d.A, d.k, d.E, Ep, bits, w.err, w.block_base,
                        (int32_t)d.T, shared, d.bm_log2, w.offsets, w.tiles, w.tile_count,
-                       w.token_map, w.inverse_map, w.row_weight);
+                       w.token_map, w.inverse_map, w.row_weight, InputF32{});
     return launch_check("grouped schedule rows");
   }
   hipLaunchKernelGGL(sched_scan_kernel, dim3(1), dim3(1024), 0, st, w.block_base, (int32_t)d.nb,
@@ -1425,6 +1445,7 @@ struct LayerCall {
   bool routed_f32 = false;      // RunLayer output: f32 routed sum, no shared expert
   hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   GemmCapture cap{nullptr, nullptr};  // optional f32 intermediates
+  InputF32 input{nullptr, nullptr, 0};  // an f32 input, converted into x
 };
 
 static int record(hipEvent_t e, hipStream_t st) {
@@ -1512,7 +1533,8 @@ static int prefill_layer(const aima_moe_layer& L, const uint16_t* x, const uint1
                          const LayerCall& call = LayerCall{}) {
   int rc = record(call.ev[0], st);
   if (rc != AIMA_OK) return rc;
-  rc = launch_schedule(ids, call.stride ? call.stride : d.k, weights, d, w, !call.routed_f32, st);
+  rc = launch_schedule(ids, call.stride ? call.stride : d.k, weights, d, w, !call.routed_f32,
+                       call.input, st);
   if (rc != AIMA_OK) return rc;
   if ((rc = record(call.ev[1], st)) != AIMA_OK) return rc;
   rc = launch_gemm<true>(L, x, d, w, call.cap, st);
@@ -1672,11 +1694,8 @@ extern "C" int aima_moe_grouped_prefill_ex(const aima_moe_layer* layer, const vo
   call.cap = GemmCapture{opt.swiglu_f32, opt.contributions_f32};
   const uint16_t* x16 = static_cast<const uint16_t*>(x);
   if (opt.input_f32) {
-    const int64_t n8 = tokens * layer->hidden / 8;
-    hipLaunchKernelGGL(f32_to_f16_kernel, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, st,
-                       static_cast<const float4*>(x), n8, reinterpret_cast<u32x4*>(w.x16));
-    rc = launch_check("moe_grouped_prefill_ex input conversion");
-    if (rc != AIMA_OK) return rc;
+    call.input = InputF32{static_cast<const float4*>(x), reinterpret_cast<u32x4*>(w.x16),
+                          tokens * layer->hidden / 8};
     x16 = w.x16;
   }
   return prefill_layer(*layer, x16, residual, topk, weights, out, d, w, st, nullptr,
@@ -1818,7 +1837,7 @@ extern "C" int aima_grouped_schedule(const int32_t* ids, const float* weights, i
   }
   AIMA_REQUIRE(aligned(workspace, 256), "grouped_schedule: workspace must be 256-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_schedule(ids, k, weights, d, w, true, st);
+  int rc = launch_schedule(ids, k, weights, d, w, true, InputF32{}, st);
   if (rc != AIMA_OK) return rc;
   AIMA_HIP(hipMemcpyAsync(offsets, w.offsets, (size_t)experts * 4, hipMemcpyDeviceToDevice, st));
   AIMA_HIP(hipMemcpyAsync(token_map, w.token_map, (size_t)d.A * 4, hipMemcpyDeviceToDevice, st));

@@ -369,3 +369,18 @@ def test_router_selection_ties(pkg, dev, E, k):
     ref_ids, ref_w = oracle.router_topk_tokens(logits, k)
     assert np.array_equal(ids.cpu().numpy(), ref_ids)
     assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")
+
+
+@pytest.mark.parametrize("T,H", [(1, 512), (128, 768), (129, 512), (700, 256)])
+def test_prefill_f32_input_conversion(pkg, dev, T, H):
+    """An f32 input is rounded to f16 by spare blocks of the schedule's first
+    launch (one-launch schedules up to 1024 assignments, and above; partial
+    last blocks): the bits of the f16 input's run."""
+    layer = pkg.synth.moe_layer(hidden=H, inter=128, experts=16, seed=700 + H, device=dev)
+    g = torch.Generator(device=dev)
+    g.manual_seed(T)
+    x = torch.randn((T, H), generator=g, device=dev)
+    ids, w = pkg.select_router_topk(pkg.synth.router_logits(T, 16, T, dev), 8)
+    a = pkg.grouped_moe_prefill_routed(layer, x, ids, w)
+    b = pkg.grouped_moe_prefill_routed(layer, x.half(), ids, w)
+    assert torch.equal(a, b)
