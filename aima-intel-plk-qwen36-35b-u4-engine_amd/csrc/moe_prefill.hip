@@ -952,7 +952,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
 // ---------------------------------------------------------------------------
 // down GEMM with the tile's token rows resident
 // ---------------------------------------------------------------------------
-// K = inter <= 512: 128 token rows of a tile fit in LDS for the whole K
+// K = inter = 512: 128 token rows of a tile fit in LDS for the whole K
 // (128 KB).  A block of 8 waves loads them once and computes a range of
 // output columns against them, 64 columns of a wave at a time (two 32-row MFMA
 // operands, so each token operand read from LDS feeds two MFMAs).  After the
@@ -969,13 +969,13 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
 // inter 512): 427 us a layer, grouped_gemm_kernel 490 (same box; MFMA-bound
 // 270 at the rate of a large f16 product).
 constexpr int kDownRows = 128;
-constexpr int kDownMaxGroups = 4;
-constexpr int kDownTokens = kDownRows * kDownMaxGroups * 256;  // bytes of LDS
+constexpr int kDownGroups = 4;  // quantization groups along K
+constexpr int kDownTokens = kDownRows * kDownGroups * 256;  // bytes of LDS
 constexpr int kDownChunk = 64;                                 // columns of a wave at a time
 
 struct DownTile {
   int64_t row0;
-  int e, rows, GK, chunk0, chunks;  // first column chunk of this wave, end of the block's
+  int e, rows, chunk0, chunks;  // first column chunk of this wave, end of the block's
 };
 
 template <int MB, bool CAP>
@@ -987,8 +987,9 @@ __device__ __forceinline__ void down_tile(const DownTile& t, const aima_moe_laye
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, hh = lane >> 5;
-  const int GK = t.GK;
-  const int64_t H = L.hidden, K = L.inter;
+  constexpr int GK = kDownGroups;
+  constexpr int64_t K = 128 * GK;
+  const int64_t H = L.hidden;
   const bool routed = t.e < L.experts;
   const aima_u4_tensor& W = routed ? L.down : L.shared_down;
   const uint32_t lds0 = lds_addr(smem);
@@ -998,16 +999,14 @@ __device__ __forceinline__ void down_tile(const DownTile& t, const aima_moe_laye
   // 4 q .. 4 q + 3, piece p of row r in slot p ^ (r & 15)
   const void* base = uniform_ptr(act);
 #pragma unroll
-  for (int g = 0; g < kDownMaxGroups; ++g) {
-    if (g < GK) {
+  for (int g = 0; g < GK; ++g) {
 #pragma unroll
-      for (int i = 0; i < MB; ++i) {
-        const int r = 4 * (wave + 8 * i) + (lane >> 4);
-        const int64_t grow = t.row0 + (r < t.rows ? r : 0);
-        const int piece = (lane & 15) ^ (r & 15);
-        lds_load16(base, (uint32_t)((grow * K + g * 128 + piece * 8) * 2),
-                   lds0 + (uint32_t)(g * kGroup + (wave + 8 * i) * 1024));
-      }
+    for (int i = 0; i < MB; ++i) {
+      const int r = 4 * (wave + 8 * i) + (lane >> 4);
+      const int64_t grow = t.row0 + (r < t.rows ? r : 0);
+      const int piece = (lane & 15) ^ (r & 15);
+      lds_load16(base, (uint32_t)((grow * K + g * 128 + piece * 8) * 2),
+                 lds0 + (uint32_t)(g * kGroup + (wave + 8 * i) * 1024));
     }
   }
 
@@ -1158,7 +1157,6 @@ __global__ __launch_bounds__(512, 2) void grouped_down_kernel(
   t.e = tiles[4 * mt + 0];
   t.row0 = tiles[4 * mt + 1] + half * kDownRows;
   t.rows = min(kDownRows, tile_rows - half * kDownRows);
-  t.GK = L.inter >> 7;
   if (t.rows <= 32) {
     const ThinArgs a{act, tiles, tile_count, nullptr, row_weight, A, 0,
                      nullptr, contrib, nullptr, cap.contrib32};
@@ -1460,14 +1458,23 @@ static bool thin_vectors(int64_t K, const aima_u4_tensor* const (&w)[4]) {
   return ok;
 }
 
+// 128-row halves of the tiles, at least.
+static int64_t down_halves(const PrefillDims& d) {
+  return (d.A + d.T + kDownRows - 1) / kDownRows;
+}
+
 // Whether the down GEMM keeps a tile's token rows in LDS
-// (grouped_down_kernel): they fit, and the tiles are tall enough that loading
-// them once pays.  Per call (hidden 2048, inter 512, 256 experts, k = 8),
-// resident against grouped_gemm_kernel: T = 777 (24 assignments per expert)
-// 190 against 186 us, T = 1200 (37) 233 against 240, T = 2048 273 against 292
-// (skewed 226 either way), T = 4096 378 against 390.
+// (grouped_down_kernel): 4 quantization groups of them (what fits, and enough
+// work to load them for: at inter 256 and 384 it measured 5 to 9 % a call
+// slower up to T = 8000), tiles taller than thin ones, and a block and a
+// quarter per CU.  Per call (hidden 2048, inter 512), resident against
+// grouped_gemm_kernel: 94 blocks (60 experts, k = 2, T = 1000) 96.1 against
+// 92.4 us, 281 (T = 3000) 127.1 against 125.0; 337 (256 experts, k = 8,
+// T = 1200) 230 against 236, T = 2048 270 against 283 (skewed 226 either way),
+// T = 3000 314 against 343.
 static bool down_rows_resident(const PrefillDims& d) {
-  return d.I <= 128 * kDownMaxGroups && d.A > 32 * (int64_t)d.E;
+  const int64_t splits = (d.H + 8 * kDownChunk - 1) / (8 * kDownChunk);
+  return d.I == 128 * kDownGroups && d.A > 32 * (int64_t)d.E && down_halves(d) * splits >= 320;
 }
 
 // Its column chunks per block: 8 (one per wave) until 16 still leave six
@@ -1475,8 +1482,7 @@ static bool down_rows_resident(const PrefillDims& d) {
 // either way; two layers of T = 16384: 2471 us with 16, 2538 with 8; T = 4096
 // 405 and 378.
 static int down_chunks(const PrefillDims& d) {
-  const int64_t halves = (d.A + d.T + kDownRows - 1) / kDownRows;
-  return halves * (d.H / (2 * 8 * kDownChunk)) >= 6 * 256 ? 16 : 8;
+  return down_halves(d) * (d.H / (2 * 8 * kDownChunk)) >= 6 * 256 ? 16 : 8;
 }
 
 // One grouped GEMM of the layer over the schedule's tiles: 16-row tiles in

@@ -305,22 +305,23 @@ def test_prefill_thin_tiles(pkg, dev, H, I, experts, shift):
     assert_parity(f16_to_f32(out), ref, what=f"thin tiles H={H} I={I} E={experts}")
 
 
-@pytest.mark.parametrize("H,I", [(256, 128), (768, 256), (512, 384), (1024, 512)])
+@pytest.mark.parametrize("H,reps,more", [(2048, 3, 700), (768, 6, 1300)])
 @pytest.mark.parametrize("capture", [False, True])
-def test_prefill_resident_down_rows(pkg, dev, H, I, capture):
-    """The down GEMM that keeps a tile's token rows in LDS (inter <= 512, over
-    32 assignments per expert): remainders around each 32-row block of both
-    128-row halves, thin halves, and column counts that leave waves without a
-    chunk (256, 768) or fill whole blocks.  With the f32 copies requested, the
+def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture):
+    """The down GEMM that keeps a tile's token rows in LDS (inter 512, over 32
+    assignments per expert, at least 320 blocks): remainders around each 32-row
+    block of both 128-row halves, thin halves, and a column count that leaves
+    waves of a block without a chunk (768).  With the f32 copies requested, the
     f16 contributions are those values rounded.  Tolerance as the other
     prefill tests."""
-    counts = [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 256, 289]
+    I = 512
+    counts = [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 256, 289] * reps + [more]
     layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=len(counts), seed=400 + H, device=dev)
     mw = moe_to_oracle(layer)
     ids = np.repeat(np.arange(len(counts)), counts).astype(np.int32)
     ids = np.random.default_rng(H + I).permutation(ids)[:, None].copy()
     T = len(ids)
-    assert T > 32 * len(counts)
+    assert T > 32 * len(counts) and -(-2 * T // 128) * -(-H // 512) >= 320
     x = pkg.synth.activations(T, H, 401, dev)
     w = torch.rand((T, 1), device=dev) + 0.5
     d_ids = torch.from_numpy(ids).to(dev)
