@@ -2,16 +2,23 @@
 // expert), where the packed weights and their dequantization, not the matrix
 // cores, set the time.
 //
-// The weights stay integers: a nibble masked in place is an f16 subnormal
-// (q * 2^-24 from the low nibble of a byte, q * 2^-20 from the high one; the
-// matrix cores keep f16 subnormals), so the eight nibbles of a word cost five
-// VALU instructions and no rounding (f16 (q - z) * s operands: 17 and one).
-// Low and high nibbles go to separate accumulators, and each 128-wide
-// quantization group is folded into the f32 result as
-//   acc += s * ((lo + hi / 16) - z * X),   X = sum of the group's activations
-// with X from the same matrix cores (an operand of equal weights).  The 2^24
-// is multiplied in at the end.  Error of a layer's output against 64 bits:
-// 3.8e-4 (f16 operands: 4.9e-4; the rest is the f16 intermediates).
+// The weights stay integers: a code shifted to bits 4..7 of a half is an f16
+// subnormal (q * 2^-20; the matrix cores keep f16 subnormals), so the eight
+// nibbles of a word cost seven VALU instructions and no rounding (f16
+// (q - z) * s operands: 17 and one).  Each 128-wide quantization group is
+// folded into the f32 result as
+//   acc += s * (sum(q 2^-20 x) - z 2^-20 * X),   X = sum(x)
+// with X from the same matrix cores (an operand of ones); the 2^20 is
+// multiplied in at the end.  Error of a layer's output against 64 bits: 3.6e-4
+// (f16 operands: 4.9e-4; the rest is the f16 intermediates).  The place of the
+// code matters: the matrix cores align a product by its operands' nominal
+// exponents, so a small subnormal's sums lose their low bits, all to one side.
+// Nibbles masked in place (q * 2^-24 and q * 2^-20, X from operands of 2^-24)
+// cost five instructions, but the outputs' mean was off by 7.6e-5 of their
+// size (here below 1e-6), which the next layer's weights enlarge: two layers,
+// T = 30: 1.04e-3 off, f16 operands 8.7e-4, here 7.0e-4.  Codes as the normal
+// values 1 + q / 16 (eight instructions) gave the same 7.0e-4 and were slower
+// (T = 96 113 against 111 us a call, T = 2048 skewed 223 against 215).
 //
 // A block of NW waves owns one tile and 32 NW weight rows (gate/up: 16 NW
 // gate and the matching 16 NW up rows).  v_mfma_f32_16x16x32_f16: the tokens
@@ -75,6 +82,10 @@ __device__ __forceinline__ void thin_store_piece(const u32x4 x0, const u32x4 x1,
   *reinterpret_cast<u32x4*>(row + ((piece ^ (r & 15)) * 16)) = lo;
   *reinterpret_cast<u32x4*>(row + (((piece + 1) ^ (r & 15)) * 16)) = hi;
 }
+
+// Codes in bits 4..7 of each half of v as f16 values q * 2^-20.
+__device__ __forceinline__ uint32_t thin_codes(uint32_t v) { return v & 0x00F000F0u; }
+constexpr float kThinUnit = 0x1p-20f;
 
 // Scales and zero points of one weight row for a turn's 4 groups.  V4: one
 // 8-byte and one 2-byte load (whole turns, aligned rows); else value by value.
@@ -217,7 +228,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[h][b] = f32x4{};
-  const u32x4 ones_bits{0x00010001u, 0x00010001u, 0x00010001u, 0x00010001u};  // 2^-24
+  const u32x4 ones_bits{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
   const f16x8 ones = __builtin_bit_cast(f16x8, ones_bits);
 
   // one group: its token rows at grp, this wave's weights wg, group i of the turn
@@ -243,24 +254,24 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
         const uint32_t v0 = wg[h][2 * m], v1 = wg[h][2 * m + 1];
-        const uint32_t u0 = v0 >> 8, u1 = v1 >> 8;
-        const u32x4 l{v0 & 0x000F000Fu, u0 & 0x000F000Fu, v1 & 0x000F000Fu, u1 & 0x000F000Fu};
-        const u32x4 t{v0 & 0x00F000F0u, u0 & 0x00F000F0u, v1 & 0x00F000F0u, u1 & 0x00F000F0u};
+        const u32x4 l{thin_codes(v0 << 4), thin_codes(v0 >> 4), thin_codes(v1 << 4),
+                      thin_codes(v1 >> 4)};
+        const u32x4 t{thin_codes(v0), thin_codes(v0 >> 8), thin_codes(v1),
+                      thin_codes(v1 >> 8)};
         lo[m] = __builtin_bit_cast(f16x8, l);
         hi[m] = __builtin_bit_cast(f16x8, t);
       }
-      const float s = sz[h].scale(i), z = sz[h].zero(i);
+      const float s = sz[h].scale(i), z = sz[h].zero(i) * kThinUnit;
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        f32x4 al = f32x4{}, ah = f32x4{};
+        f32x4 al = f32x4{};
         al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][0], lo[0], al, 0, 0, 0);
-        ah = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][1], hi[0], ah, 0, 0, 0);
+        al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][1], hi[0], al, 0, 0, 0);
         al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][2], lo[1], al, 0, 0, 0);
-        ah = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][3], hi[1], ah, 0, 0, 0);
+        al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][3], hi[1], al, 0, 0, 0);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          float t = fmaf(ah[j], 0.0625f, al[j]);
-          t = fmaf(-z, X[b][j], t);
+          const float t = fmaf(-z, X[b][j], al[j]);
           acc[h][b][j] = fmaf(s, t, acc[h][b][j]);
         }
       }
@@ -326,7 +337,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
     for (int j = 0; j < 4; ++j) {
       const int m = b * 16 + 4 * q + j;
       if (GATEUP) {
-        const float g = acc[0][b][j] * 16777216.0f, u = acc[1][b][j] * 16777216.0f;
+        const float g = acc[0][b][j] * (1.0f / kThinUnit), u = acc[1][b][j] * (1.0f / kThinUnit);
         const float o = as_f32_value(g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g)));
         stage[m * (kCols + 8) + n] = f2h(o);
         if (CAP && a.act32 && m < rows) a.act32[(row0 + m) * ld + col0 + n] = o;
@@ -334,7 +345,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
         const float wt = routed && m < rows ? a.row_weight[row0 + m] : 1.0f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const float o = as_f32_value(wt * (acc[h][b][j] * 16777216.0f));
+          const float o = as_f32_value(wt * (acc[h][b][j] * (1.0f / kThinUnit)));
           stage[m * (kCols + 8) + 16 * h + n] = f2h(o);
           if (CAP && a.contrib32 && m < rows) a.contrib32[(row0 + m) * ld + col0 + 16 * h + n] = o;
         }

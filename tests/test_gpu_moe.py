@@ -305,6 +305,26 @@ def test_prefill_thin_tiles(pkg, dev, H, I, experts, shift):
     assert_parity(f16_to_f32(out), ref, what=f"thin tiles H={H} I={I} E={experts}")
 
 
+@pytest.mark.parametrize("H,I", [(1024, 256), (2048, 768)])
+def test_prefill_thin_tiles_unbiased(pkg, dev, H, I):
+    """A thin tile's result is off by roundings, not to one side: an offset
+    common to all outputs passes through the next layers' weights (whose mean
+    is not zero) enlarged.  The outputs' errors are roundings of the f16
+    intermediates, below 2^-11 of the output's size and independent, so their
+    mean over n outputs lies within 6 * 2^-11 / sqrt(n) of zero (1.7e-5 and
+    1.2e-5 of the outputs' size)."""
+    layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=60, seed=320 + H, device=dev)
+    T, k = 30, 2
+    x = pkg.synth.activations(T, H, 321, dev).float()
+    ids, w = pkg.select_router_topk(pkg.synth.router_logits(T, 60, 322, dev), k)
+    out = pkg.grouped_moe_prefill_routed(layer, x, ids, w, expert_used_count=k)
+    torch.cuda.synchronize()
+    ref = oracle.moe_routed_tokens(moe_to_oracle(layer), x.cpu().numpy(), ids.cpu().numpy(),
+                                   w.cpu().numpy(), threads=THREADS).astype(np.float64)
+    off = (out.cpu().numpy() - ref).mean() / np.sqrt((ref ** 2).mean())
+    assert abs(off) <= 6 * 2.0 ** -11 / np.sqrt(ref.size)
+
+
 @pytest.mark.parametrize("H,reps,more", [(2048, 3, 700), (768, 6, 1300)])
 @pytest.mark.parametrize("capture", [False, True])
 def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture):
