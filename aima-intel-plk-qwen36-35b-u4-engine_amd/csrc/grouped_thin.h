@@ -35,8 +35,10 @@
 // Bound: the weights' bytes.  T = 96 over 256 experts (hidden 2048, inter
 // 512; 289 and 145 MB of weights): gate/up 57 us, down 35 (5.1 and 4.1 TB/s;
 // a bare read in the same pattern reaches 6.1), against 90 and 63 us with
-// f16 operands in 512-thread blocks.  Without its arithmetic the kernel takes
-// 55 and 31 us: first loads and the last blocks are the rest.
+// f16 operands in 512-thread blocks, both with the nibbles masked in place; the
+// two shifts more per word add 5 us to a call (164 us with f16 operands, 110).
+// Without its arithmetic the kernel takes 55 and 31 us: first loads and the
+// last blocks are the rest.
 #ifndef AIMA_GROUPED_THIN_H_
 #define AIMA_GROUPED_THIN_H_
 
