@@ -2,23 +2,21 @@
 // expert), where the packed weights and their dequantization, not the matrix
 // cores, set the time.
 //
-// The weights stay integers: a code shifted to bits 4..7 of a half is an f16
-// subnormal (q * 2^-20; the matrix cores keep f16 subnormals), so the eight
-// nibbles of a word cost seven VALU instructions and no rounding (f16
-// (q - z) * s operands: 17 and one).  Each 128-wide quantization group is
-// folded into the f32 result as
-//   acc += s * (sum(q 2^-20 x) - z 2^-20 * X),   X = sum(x)
-// with X from the same matrix cores (an operand of ones); the 2^20 is
-// multiplied in at the end.  Error of a layer's output against 64 bits: 3.6e-4
-// (f16 operands: 4.9e-4; the rest is the f16 intermediates).  The place of the
-// code matters: the matrix cores align a product by its operands' nominal
-// exponents, so a small subnormal's sums lose their low bits, all to one side.
-// Nibbles masked in place (q * 2^-24 and q * 2^-20, X from operands of 2^-24)
-// cost five instructions, but the outputs' mean was off by 7.6e-5 of their
-// size (here below 1e-6), which the next layer's weights enlarge: two layers,
-// T = 30: 1.04e-3 off, f16 operands 8.7e-4, here 7.0e-4.  Codes as the normal
-// values 1 + q / 16 (eight instructions) gave the same 7.0e-4 and were slower
-// (T = 96 113 against 111 us a call, T = 2048 skewed 223 against 215).
+// The weights enter as the integers q - z, exact in f16: a code OR-ed into
+// bits 0..3 of 0x6400 is 1024 + q, into bits 4..7 of 0x5400 64 + q, and one
+// subtraction leaves q - z, nine VALU instructions for the eight nibbles of a
+// word and no rounding (f16 (q - z) * s operands: 17 and one).  Each 128-wide
+// quantization group is folded into the f32 result as
+//   acc += s * sum((q - z) x)
+// Error of a layer's output against 64 bits: 3.6e-4 (f16 operands: 4.9e-4; the
+// rest is the f16 intermediates), with a few channels 2^4 .. 2^12 times the
+// rest too (3.0e-4 and 4.6e-4 with f32 outputs).  An infinite x keeps its sign
+// through q - z, as in the products with (q - z) * s.
+// The z must be subtracted before the product: sum(q x) - z sum(x), with the
+// codes alone as (subnormal) operands, takes two instructions less a word, but
+// an infinite x makes it inf - inf, sum(x) takes MFMAs of its own, and its
+// extra fold and registers cost more than they save: T = 777 (24 rows an
+// expert) 168 us a call against 157 here, T = 96 110.5 against 110.3.
 //
 // A block of NW waves owns one tile and 32 NW weight rows (gate/up: 16 NW
 // gate and the matching 16 NW up rows).  v_mfma_f32_16x16x32_f16: the tokens
@@ -33,12 +31,10 @@
 // the current ones are used.
 //
 // Bound: the weights' bytes.  T = 96 over 256 experts (hidden 2048, inter
-// 512; 289 and 145 MB of weights): gate/up 57 us, down 35 (5.1 and 4.1 TB/s;
-// a bare read in the same pattern reaches 6.1), against 90 and 63 us with
-// f16 operands in 512-thread blocks, both with the nibbles masked in place; the
-// two shifts more per word add 5 us to a call (164 us with f16 operands, 110).
-// Without its arithmetic the kernel takes 55 and 31 us: first loads and the
-// last blocks are the rest.
+// 512; about 245 experts active: 267 and 133 MB of weights): gate/up 62.6 us,
+// down 37.0 (4.3 and 3.6 TB/s, in a kernel trace; a bare read in the same
+// pattern reaches 6.1).  The call takes 108.5 us; with f16 (q - z) * s operands
+// in 512-thread blocks and three schedule launches it took 160.
 #ifndef AIMA_GROUPED_THIN_H_
 #define AIMA_GROUPED_THIN_H_
 
@@ -85,9 +81,35 @@ __device__ __forceinline__ void thin_store_piece(const u32x4 x0, const u32x4 x1,
   *reinterpret_cast<u32x4*>(row + (((piece + 1) ^ (r & 15)) * 16)) = hi;
 }
 
-// Codes in bits 4..7 of each half of v as f16 values q * 2^-20.
-__device__ __forceinline__ uint32_t thin_codes(uint32_t v) { return v & 0x00F000F0u; }
-constexpr float kThinUnit = 0x1p-20f;
+// The halves 0x6400 and 0x5400 in VGPRs (as u4_magic): a code OR-ed into bits
+// 0..3 or 4..7 of them is the f16 value 1024 + q or 64 + q.
+struct ThinMagic {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ ThinMagic thin_magic() {
+  ThinMagic m{u4_magic(), 0x54005400u};
+  asm volatile("" : "+v"(m.hi));
+  return m;
+}
+
+// 1024 + z and 64 + z of one weight row and group, and the exact operands
+// q - z of a word (k 0..7): `lo` holds k 0, 4, 2, 6 (bits 0..3 of each byte),
+// `hi` k 1, 5, 3, 7.
+struct ThinZero {
+  f16x2 lo, hi;
+};
+__device__ __forceinline__ ThinZero thin_zero(uint32_t z, const ThinMagic& m) {
+  const uint32_t zz = z * 0x00010001u;
+  return ThinZero{as_h2(zz | m.lo), as_h2((zz << 4) | m.hi)};
+}
+__device__ __forceinline__ void thin_word(uint32_t v, const ThinZero& z, const ThinMagic& m,
+                                          uint32_t (&lo)[2], uint32_t (&hi)[2]) {
+  const uint32_t v8 = v >> 8;
+  lo[0] = h2_bits(as_h2((v & 0x000F000Fu) | m.lo) - z.lo);
+  hi[0] = h2_bits(as_h2((v & 0x00F000F0u) | m.hi) - z.hi);
+  lo[1] = h2_bits(as_h2((v8 & 0x000F000Fu) | m.lo) - z.lo);
+  hi[1] = h2_bits(as_h2((v8 & 0x00F000F0u) | m.hi) - z.hi);
+}
 
 // Scales and zero points of one weight row for a turn's 4 groups.  V4: one
 // 8-byte and one 2-byte load (whole turns, aligned rows); else value by value.
@@ -106,7 +128,7 @@ struct ThinSz {
     const f16x2 v = as_h2(s[i >> 1]);
     return i & 1 ? (float)v.y : (float)v.x;
   }
-  __device__ __forceinline__ float zero(int i) const { return (float)((z >> (4 * i)) & 0xfu); }
+  __device__ __forceinline__ uint32_t zero(int i) const { return (z >> (4 * i)) & 0xfu; }
 };
 template <>
 struct ThinSz<false> {
@@ -121,8 +143,8 @@ struct ThinSz<false> {
     }
   }
   __device__ __forceinline__ float scale(int i) const { return h2f((uint16_t)s[i]); }
-  __device__ __forceinline__ float zero(int i) const {
-    return (float)((z[i] >> ((z[i] >> 16) * 4)) & 0xfu);
+  __device__ __forceinline__ uint32_t zero(int i) const {
+    return (z[i] >> ((z[i] >> 16) * 4)) & 0xfu;
   }
 };
 
@@ -230,8 +252,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[h][b] = f32x4{};
-  const u32x4 ones_bits{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
-  const f16x8 ones = __builtin_bit_cast(f16x8, ones_bits);
+  const ThinMagic magic = thin_magic();
 
   // one group: its token rows at grp, this wave's weights wg, group i of the turn
   auto group = [&](const uint8_t* grp, const u32x4 (&wg)[2], int i) {
@@ -242,28 +263,19 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
       for (int p = 0; p < 4; ++p)
         tf[b][p] = *reinterpret_cast<const f16x8*>(grp + (b * 16 + n) * 256 +
                                                    (((q * 4 + p) ^ n) * 16));
-    f32x4 X[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      f32x4 x = f32x4{};
-#pragma unroll
-      for (int p = 0; p < 4; ++p) x = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][p], ones, x, 0, 0, 0);
-      X[b] = x;
-    }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      const ThinZero z = thin_zero(sz[h].zero(i), magic);
       f16x8 lo[2], hi[2];
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
-        const uint32_t v0 = wg[h][2 * m], v1 = wg[h][2 * m + 1];
-        const u32x4 l{thin_codes(v0 << 4), thin_codes(v0 >> 4), thin_codes(v1 << 4),
-                      thin_codes(v1 >> 4)};
-        const u32x4 t{thin_codes(v0), thin_codes(v0 >> 8), thin_codes(v1),
-                      thin_codes(v1 >> 8)};
-        lo[m] = __builtin_bit_cast(f16x8, l);
-        hi[m] = __builtin_bit_cast(f16x8, t);
+        uint32_t l0[2], l1[2], h0[2], h1[2];
+        thin_word(wg[h][2 * m], z, magic, l0, h0);
+        thin_word(wg[h][2 * m + 1], z, magic, l1, h1);
+        lo[m] = __builtin_bit_cast(f16x8, (u32x4{l0[0], l0[1], l1[0], l1[1]}));
+        hi[m] = __builtin_bit_cast(f16x8, (u32x4{h0[0], h0[1], h1[0], h1[1]}));
       }
-      const float s = sz[h].scale(i), z = sz[h].zero(i) * kThinUnit;
+      const float s = sz[h].scale(i);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         f32x4 al = f32x4{};
@@ -272,10 +284,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
         al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][2], lo[1], al, 0, 0, 0);
         al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tf[b][3], hi[1], al, 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float t = fmaf(-z, X[b][j], al[j]);
-          acc[h][b][j] = fmaf(s, t, acc[h][b][j]);
-        }
+        for (int j = 0; j < 4; ++j) acc[h][b][j] = fmaf(s, al[j], acc[h][b][j]);
       }
     }
   };
@@ -339,7 +348,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
     for (int j = 0; j < 4; ++j) {
       const int m = b * 16 + 4 * q + j;
       if (GATEUP) {
-        const float g = acc[0][b][j] * (1.0f / kThinUnit), u = acc[1][b][j] * (1.0f / kThinUnit);
+        const float g = acc[0][b][j], u = acc[1][b][j];
         const float o = as_f32_value(g * u * __builtin_amdgcn_rcpf(1.0f + __expf(-g)));
         stage[m * (kCols + 8) + n] = f2h(o);
         if (CAP && a.act32 && m < rows) a.act32[(row0 + m) * ld + col0 + n] = o;
@@ -347,7 +356,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
         const float wt = routed && m < rows ? a.row_weight[row0 + m] : 1.0f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const float o = as_f32_value(wt * (acc[h][b][j] * (1.0f / kThinUnit)));
+          const float o = as_f32_value(wt * acc[h][b][j]);
           stage[m * (kCols + 8) + 16 * h + n] = f2h(o);
           if (CAP && a.contrib32 && m < rows) a.contrib32[(row0 + m) * ld + col0 + 16 * h + n] = o;
         }

@@ -10,8 +10,9 @@
 // 2. Grouped gate/up GEMM (MFMA v_mfma_f32_32x32x16_f16): per tile, the token
 //    rows are gathered into LDS; each wave dequantizes its own 32 weight rows
 //    straight into MFMA operands as f16 (q - z) * s and multiplies them with
-//    every token row of the tile; tiles of at most 32 rows multiply the integer
-//    codes instead (grouped_thin.h).  The SwiGLU epilogue writes f16 [rows][I].
+//    every token row of the tile; tiles of at most 32 rows multiply the integers
+//    q - z instead and scale the sums (grouped_thin.h).  The SwiGLU epilogue
+//    writes f16 [rows][I].
 // 3. Grouped down GEMM, same structure over K = I; its output rows times their
 //    router weights (1 for the shared expert) are the contributions, written as
 //    f16 [rows][H].
@@ -856,10 +857,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
 
   // Tiles of one 32-row block: their time is the dequantization of weights
   // that feed a single MFMA each, so they take the integer operands of
-  // thin_tile.  Against f16 operands on this block's own path (T = 777,
-  // uniform routing): 192 against 213 us per call; T = 900, skewed: 140
-  // against 159; T = 2048, skewed (101 of 141 experts have at most 32 rows):
-  // 238 against 252.
+  // thin_tile.  T = 777, uniform routing: 157 us per call (f16 operands on this
+  // block's own path, with one schedule launch more: 182).
   if (tiles[4 * mt + 2] <= 32) {
     const ThinArgs a{src, tiles, tile_count, token_map, row_weight, A, ntiles_n,
                      act_out, contrib_out, cap.act32, cap.contrib32};

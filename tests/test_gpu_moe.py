@@ -405,3 +405,91 @@ def test_prefill_f32_input_conversion(pkg, dev, T, H):
     a = pkg.grouped_moe_prefill_routed(layer, x, ids, w)
     b = pkg.grouped_moe_prefill_routed(layer, x.half(), ids, w)
     assert torch.equal(a, b)
+
+
+def _dequant_f64(w):
+    q = w.qweight.cpu().numpy().reshape(w.rows, w.k // 2)
+    s = w.scale.cpu().view(torch.uint16).numpy().reshape(w.rows, -1)
+    z = w.zp.cpu().numpy().reshape(-1)
+    return torch.from_numpy(oracle.u4_dequant(q, s, z, w.rows, w.k, w.group)).double()
+
+
+def _expert_f64(layer, x):
+    """SwiGLU and down rows of a one-expert layer in float64, the SwiGLU rows
+    rounded to f16 in between."""
+    gu = _dequant_f64(layer.gate_up) @ x.double().cpu().T
+    g, u = gu[:layer.inter], gu[layer.inter:]
+    act = (g * torch.sigmoid(g) * u).T
+    return act, act.half().double() @ _dequant_f64(layer.down).T
+
+
+def _same_class(got, ref):
+    """The same elements are +inf, -inf and NaN."""
+    return all(torch.equal(f(got.double().cpu()), f(ref))
+               for f in (torch.isposinf, torch.isneginf, torch.isnan))
+
+
+@pytest.mark.parametrize("rows", [5, 12, 20, 40])
+@pytest.mark.parametrize("inter", [128, 512])
+def test_prefill_infinities(pkg, dev, rows, inter):
+    """An infinite activation and a SwiGLU value past f16's range reach the
+    result as +-inf or NaN just where (q - z) * s * x gives them, in every
+    tile height: 16-row tiles (5), thin tiles of one and two 16-row blocks (12,
+    20) and a taller one (40)."""
+    layer = pkg.synth.moe_layer(hidden=512, inter=inter, experts=1, seed=60 + rows, device=dev)
+    ids = torch.zeros((rows, 1), dtype=torch.int32, device=dev)
+    w = torch.ones((rows, 1), device=dev)
+    x = pkg.synth.activations(rows, 512, 61, dev)
+    x[0, 77] = float("inf")
+    x[rows - 1, 300] = -float("inf")
+    x[2, 5], x[2, 6] = float("inf"), -float("inf")
+    cap = {}
+    pkg.grouped_moe_prefill_routed(layer, x, ids, w, expert_used_count=1, capture_f32=cap)
+    act, _ = _expert_f64(layer, x)
+    assert torch.isinf(act).any() and torch.isfinite(act[1]).all()
+    assert _same_class(cap["swiglu_f32"], act)
+    # one intermediate column of a few rows past 65504 (x = +-400 against a
+    # gate and an up row of ones), positive down weights but for one column
+    for t, code in ((layer.gate_up, 0x11), (layer.down, None)):
+        t.zp.zero_()
+        if code is not None:
+            v = t.qweight.view(2 * inter, 256)
+            v[7], v[inter + 7] = code, code
+            t.scale.view(2 * inter, -1)[7] = 1.0
+            t.scale.view(2 * inter, -1)[inter + 7] = 1.0
+    d = layer.down.qweight.view(512, inter // 2)
+    d[:, 3] = (d[:, 3] & 0x0F) | 0x10   # column 7: code 1, +inf, ...
+    d[9, 3] = d[9, 3] & 0x0F            # ... and 0, NaN, in row 9
+    x = pkg.synth.activations(rows, 512, 62, dev) * 0.01
+    x[1] = 400.0 / 512
+    x[rows - 1] = 400.0 / 512
+    out = pkg.grouped_moe_prefill_routed(layer, x, ids, w, expert_used_count=1)
+    act, ref = _expert_f64(layer, x)
+    assert torch.isposinf(act.half()[1, 7]) and torch.isfinite(act.half()[0]).all()
+    assert torch.isposinf(ref[1, 0]) and torch.isnan(ref[1, 9])
+    assert _same_class(out, ref)
+    fin = torch.isfinite(ref)
+    assert_parity(out.cpu()[fin].numpy(), ref[fin].numpy(), what=f"finite rows of {rows}")
+
+
+@pytest.mark.parametrize("rows", [12, 20, 40])
+@pytest.mark.parametrize("factor", [2.0 ** 4, 2.0 ** 8, 2.0 ** 12])
+def test_prefill_outlier_channels(pkg, dev, rows, factor):
+    """A few channels 2^4 to 2^12 times the rest cost no precision: an output
+    passes through at most four independent f16 roundings (the operands of the
+    two GEMMs, the SwiGLU value, the contribution), each at most 2^-11, so the
+    outputs are off by at most sqrt(4) * 2^-11 of their root mean square."""
+    H, I = 1024, 256
+    layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=1, seed=80 + rows, device=dev)
+    x = pkg.synth.activations(rows, H, 81, dev).float()
+    ch = torch.arange(3, H, 341, device=dev)
+    x[:, ch] *= factor
+    x = (x / (1.0 + factor * len(ch) / H ** 0.5)).half()
+    ids = torch.zeros((rows, 1), dtype=torch.int32, device=dev)
+    w = torch.ones((rows, 1), device=dev)
+    out = pkg.grouped_moe_prefill_routed(layer, x, ids, w, expert_used_count=1)
+    gu = _dequant_f64(layer.gate_up) @ x.double().cpu().T
+    g, u = gu[:I], gu[I:]
+    ref = (g * torch.sigmoid(g) * u).T @ _dequant_f64(layer.down).T
+    err = (out.double().cpu() - ref).square().mean().sqrt() / ref.square().mean().sqrt()
+    assert err <= 2.0 ** -10
