@@ -31,6 +31,7 @@ from .ops import (  # noqa: F401
     moe_stack_decode,
     moe_stack_decode_routed,
     moe_stack_prefill,
+    prefill_tiling,
     prefill_workspace_views,
     q4k_unpack,
     q4s_matvec,

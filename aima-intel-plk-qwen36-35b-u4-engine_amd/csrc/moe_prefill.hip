@@ -1484,6 +1484,11 @@ static int down_chunks(const PrefillDims& d) {
   return down_halves(d) * (d.H / (2 * 8 * kDownChunk)) >= 6 * 256 ? 16 : 8;
 }
 
+// Blocks per M tile of the gate/up GEMM.
+static int gateup_blocks(const PrefillDims& d) {
+  return d.I / (d.bm_log2 == kMinTileLog2 ? 64 : 128);
+}
+
 // One grouped GEMM of the layer over the schedule's tiles: 16-row tiles in
 // blocks of 256 threads, 256-row tiles in blocks of 512 (tile_rows_log2).
 template <bool GATEUP>
@@ -1502,7 +1507,7 @@ static int launch_gemm(const aima_moe_layer& L, const uint16_t* src, const Prefi
   const unsigned mtiles = (unsigned)round_up(d.max_tiles, 8);
   auto pick = [&](auto vec, auto gen, auto full) { return v4 ? vec : capture ? full : gen; };
   if (d.bm_log2 == kMinTileLog2) {
-    const int nt = GATEUP ? d.I / 64 : d.H / 128;
+    const int nt = GATEUP ? gateup_blocks(d) : d.H / 128;
     const ThinArgs a{src,   w.tiles,   w.tile_count, w.token_map, w.row_weight, d.A, nt,
                      w.act, w.contrib, cap.act32,    cap.contrib32};
     hipLaunchKernelGGL(pick(grouped_thin_kernel<GATEUP, true, false>,
@@ -1519,7 +1524,7 @@ static int launch_gemm(const aima_moe_layer& L, const uint16_t* src, const Prefi
                        dim3(mtiles * 2 * splits), dim3(512), 0, st, L, src, w.tiles, w.tile_count,
                        w.row_weight, d.A, splits, cpb, w.contrib, cap);
   } else {
-    const int nt = GATEUP ? d.I / 128 : d.H / 256;
+    const int nt = GATEUP ? gateup_blocks(d) : d.H / 256;
     hipLaunchKernelGGL(pick(grouped_gemm_kernel<GATEUP, true, false>,
                             grouped_gemm_kernel<GATEUP, false, false>,
                             grouped_gemm_kernel<GATEUP, false, true>),
@@ -1763,6 +1768,19 @@ extern "C" int aima_moe_prefill_workspace_views(const aima_moe_layer* layer, int
   views->contributions = w.contrib;
   views->tiles = w.tiles;
   views->tile_count = w.tile_count;
+  return AIMA_OK;
+}
+
+extern "C" int aima_moe_prefill_tiling(const aima_moe_layer* layer, int64_t tokens, int32_t k,
+                                       int32_t output_mode, int32_t* tile_rows,
+                                       int32_t* gateup_tile_blocks) {
+  AIMA_REQUIRE(layer && tile_rows && gateup_tile_blocks, "moe_prefill_tiling: null pointer");
+  AIMA_REQUIRE(tokens > 0 && k > 0, "moe_prefill_tiling: tokens and k must be positive");
+  AIMA_REQUIRE(output_mode == AIMA_PREFILL_FULL_F16 || output_mode == AIMA_PREFILL_ROUTED_F32,
+               "moe_prefill_tiling: unknown output mode");
+  const PrefillDims d = prefill_dims(layer, tokens, k);
+  *tile_rows = 1 << d.bm_log2;
+  *gateup_tile_blocks = gateup_blocks(d);
   return AIMA_OK;
 }
 

@@ -690,6 +690,15 @@ def prefill_workspace_views(layer: MoeLayerWeights, tokens: int, k: int, ws: Wor
             "tile_count": view(v.tile_count, 1, torch.int32)}
 
 
+def prefill_tiling(layer: MoeLayerWeights, tokens: int, k: int, with_shared: bool = True):
+    """(rows of a full M tile, gate/up blocks per tile) of a prefill call."""
+    rows, blocks = C.c_int32(), C.c_int32()
+    mode = _lib.AIMA_PREFILL_FULL_F16 if with_shared else _lib.AIMA_PREFILL_ROUTED_F32
+    call("aima_moe_prefill_tiling", C.byref(layer.c()), int(tokens), int(k), mode, C.byref(rows),
+         C.byref(blocks))
+    return rows.value, blocks.value
+
+
 def build_grouped_schedule(ids: torch.Tensor, router_weights: torch.Tensor, experts: int,
                            ws: Optional[Workspace] = None) -> dict:
     """Device BuildGroupedSchedule: offsets [E], token_map/inverse_map/compact_weights [T*k]."""

@@ -268,8 +268,8 @@ def test_prefill_workspace_views(pkg):
     assert base <= v.tile_count < v.offsets
 
 
-def _tiles_needed(counts, T, bm=256):
-    """Tile records the schedule writes: per expert with rows, its full 256-row
+def _tiles_needed(counts, T, bm):
+    """Tile records the schedule writes: per expert with rows, its full bm-row
     tiles and one remainder tile; the shared expert's T rows likewise."""
     n = sum(c // bm + (1 if c % bm else 0) for c in counts)
     return n + T // bm + (1 if T % bm else 0)
@@ -295,6 +295,10 @@ def test_prefill_workspace_holds_every_tile(pkg, T, k, E):
     L.call("aima_moe_prefill_workspace_views", C.byref(lc), T, k, C.c_void_p(base), C.byref(v))
     capacity = (v.token_map - v.tiles) // 16
     assert base + size >= v.contributions + (T * k + T) * 2048 * 2
+    rows, blocks = C.c_int32(), C.c_int32()
+    L.call("aima_moe_prefill_tiling", C.byref(lc), T, k, L.AIMA_PREFILL_FULL_F16, C.byref(rows),
+           C.byref(blocks))
+    assert rows.value in (16, 256) and blocks.value == 512 // (64 if rows.value == 16 else 128)
     rng = np.random.default_rng(T * 31 + k * 7 + E)
     zipf = 1.0 / np.arange(1, E + 1) ** 1.1
     routings = {
@@ -311,7 +315,7 @@ def test_prefill_workspace_holds_every_tile(pkg, T, k, E):
         ends = s["offsets"].astype(np.int64)
         counts = np.diff(np.concatenate([[0], ends]))
         assert counts.sum() == T * k
-        need = _tiles_needed(counts.tolist(), T)
+        need = _tiles_needed(counts.tolist(), T, rows.value)
         assert need <= capacity, (name, need, capacity)
 
 

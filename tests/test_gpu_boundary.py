@@ -191,6 +191,20 @@ def test_run_layer_intermediates_and_stages(pkg, dev, layer_c2):
     assert_parity(run.output.cpu().numpy(), ref, what="runtime routed")
 
 
+@pytest.mark.parametrize("T,tile,units", [(300, 16, 64), (400, 256, 128)])
+def test_run_layer_work_tiles(pkg, dev, layer_c2, T, tile, units):
+    """gateup_work_tile_count counts the blocks of the gate/up launch, in
+    16-row tiles of 64 intermediate units and in 256-row ones of 128."""
+    layer, _ = layer_c2
+    ids, w = pkg.select_router_topk(pkg.synth.router_logits(T, 256, 96, dev), 8)
+    rt = pkg.GroupedU4PrefillRuntime(dev)
+    run = rt.RunLayer(rt.LoadLayer(layer), pkg.GroupedU4PrefillInput(
+        pkg.synth.activations(T, 2048, 95, dev), ids, w.reshape(-1), capture_intermediates=True))
+    counts = np.bincount(ids.cpu().numpy().reshape(-1), minlength=256)
+    assert pkg.prefill_tiling(layer, T, 8, with_shared=False) == (tile, 512 // units)
+    assert run.gateup_work_tile_count == int((-(-counts // tile)).sum()) * (512 // units)
+
+
 @pytest.fixture(scope="module")
 def split_pair(pkg, dev, layer_c2):
     layer, mw = layer_c2
