@@ -70,19 +70,32 @@ static int64_t tile_bound(const PrefillDims& d, int64_t bm) {
   return (d.A + bm - 1) / bm + std::min<int64_t>(d.E, d.A) + (d.T + bm - 1) / bm;
 }
 
-// Tile height.  Up to 10 assignments per expert on average, most tiles are
-// thin whatever the height, and 16-row tiles in small blocks (several per CU:
-// grouped_thin_kernel) beat the 512-thread blocks of grouped_gemm_kernel:
-// T = 96 (3 per expert, hidden 2048, inter 512, 256 experts, k = 8) 108
-// against 134 us per call, T = 200 (6.3) 119 against 150, uniform routing.
-// Beyond, an expert's weights are read once per 16 rows for nothing: at 12.5
-// per expert 141 against 160 us if the routing is uniform, but 116 against
-// 109 if it is skewed, 14 per expert 124 against 110.
-static int tile_rows_log2(const PrefillDims& d) {
-  return d.A <= 10 * (int64_t)d.E ? kMinTileLog2 : 8;
+// Tile height.  16-row tiles in small blocks (several per CU:
+// grouped_thin_kernel) beat the 512-thread blocks of grouped_gemm_kernel while
+// most experts have few rows; but every 16 rows read an expert's weights
+// again.  Two limits, for the two ways of having more rows:
+// - up to 10 assignments per expert on average: uniform routing, hidden 2048,
+//   inter 512, 256 experts, k = 8, 16-row against 256-row tiles: T = 96 (3 per
+//   expert) 109 against 123 us per call, T = 320 (10) 127 against 146, T = 400
+//   (12.5) 138 against 148, but with the routed output alone 133 and 134.
+// - a bound on all rows (the shared expert's T among them), whatever the number
+//   of experts: skewed routing gives them to few experts, and the 256-row
+//   kernel takes those at a nearly constant time (one tall tile's).  Zipf 1.1,
+//   inter 512: k = 1, T = 1600 (3200 rows) 89 against 87 us, T = 2560 125
+//   against 95; k = 8, T = 300 92 against 91.  Beyond inter 512 a 16-row tile
+//   costs more and the 256-row kernel, with more blocks per tile, hardly: inter
+//   768, k = 8, T = 100 (900 rows) 72 against 66 us, T = 200 109 against 92,
+//   T = 300 140 against 102; inter 1024, hidden 4096, k = 1, T = 1900 294
+//   against 182; uniform there: inter 768, T = 150 176 against 195, T = 300
+//   192 against 205.
+static int tile_rows_log2(const PrefillDims& d, bool with_shared) {
+  const int64_t rows = d.A + (with_shared ? d.T : 0);
+  const int64_t most = d.I <= 512 ? 3200 : (13 << 16) / d.I;
+  return d.A <= 10 * (int64_t)d.E && rows <= most ? kMinTileLog2 : 8;
 }
 
-static PrefillDims prefill_dims(const aima_moe_layer* L, int64_t T, int k) {
+static PrefillDims prefill_dims(const aima_moe_layer* L, int64_t T, int k,
+                                bool with_shared = true) {
   PrefillDims d;
   d.T = T;
   d.k = k;
@@ -91,7 +104,7 @@ static PrefillDims prefill_dims(const aima_moe_layer* L, int64_t T, int k) {
   d.H = L->hidden;
   d.I = L->inter;
   d.nb = (d.A + kSchedBlock - 1) / kSchedBlock;
-  d.bm_log2 = tile_rows_log2(d);
+  d.bm_log2 = tile_rows_log2(d, with_shared);
   d.max_tiles = tile_bound(d, 1 << d.bm_log2);
   return d;
 }
@@ -1687,7 +1700,7 @@ extern "C" int aima_moe_grouped_prefill_ex(const aima_moe_layer* layer, const vo
                "below 2^30 (split the batch)");
   AIMA_REQUIRE(aligned(x, 16) && aligned(out, 16) && (!residual || aligned(residual, 16)),
                "moe_grouped_prefill_ex: x, residual and out must be 16-byte aligned");
-  const PrefillDims d = prefill_dims(layer, tokens, k);
+  const PrefillDims d = prefill_dims(layer, tokens, k, !routed);
   PrefillWs w{};
   const size_t need = prefill_ws_layout(d, WsMode::kLayer, workspace, &w);
   if (!workspace || workspace_bytes < need) {
@@ -1778,7 +1791,8 @@ extern "C" int aima_moe_prefill_tiling(const aima_moe_layer* layer, int64_t toke
   AIMA_REQUIRE(tokens > 0 && k > 0, "moe_prefill_tiling: tokens and k must be positive");
   AIMA_REQUIRE(output_mode == AIMA_PREFILL_FULL_F16 || output_mode == AIMA_PREFILL_ROUTED_F32,
                "moe_prefill_tiling: unknown output mode");
-  const PrefillDims d = prefill_dims(layer, tokens, k);
+  const PrefillDims d =
+      prefill_dims(layer, tokens, k, output_mode != AIMA_PREFILL_ROUTED_F32);
   *tile_rows = 1 << d.bm_log2;
   *gateup_tile_blocks = gateup_blocks(d);
   return AIMA_OK;

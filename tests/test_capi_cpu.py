@@ -363,3 +363,27 @@ def test_router_gemm_validation(pkg):
     args = lambda x, H: (x, 1, 64, H, p, 256, 8, C.c_float(6.1e-5), p, p, p, None, 0, None)
     assert lib.aima_router_gemm_topk(*args(p, 2040)) == L.AIMA_E_INVALID
     assert lib.aima_router_gemm_topk(*args(odd, 2048)) == L.AIMA_E_INVALID
+
+
+@pytest.mark.parametrize("H,I,E,k,shared,last", [
+    (2048, 512, 256, 8, False, 320),    # 10 assignments per expert
+    (2048, 512, 256, 8, True, 320),
+    (2048, 512, 256, 1, False, 2560),
+    (2048, 512, 256, 1, True, 1600),    # 3200 rows with the shared expert's
+    (2048, 512, 60, 1, True, 600),
+    (2048, 768, 256, 8, False, 138),    # 1109 rows
+    (2048, 768, 256, 8, True, 123),
+    (4096, 1024, 256, 1, True, 416),    # 832 rows
+])
+def test_prefill_thin_tile_rule(pkg, H, I, E, k, shared, last):
+    """The most tokens of a call in 16-row tiles: beyond, skewed routing made
+    them up to 1.7 times slower than 256-row ones."""
+    L = pkg._lib
+    lc = _fake_layer(pkg, H=H, I=I, E=E)
+    rows, blocks = C.c_int32(), C.c_int32()
+    for T, tile in ((1, 16), (last, 16), (last + 1, 256), (100000, 256)):
+        L.call("aima_moe_prefill_tiling", C.byref(lc), T, k,
+               L.AIMA_PREFILL_FULL_F16 if shared else L.AIMA_PREFILL_ROUTED_F32, C.byref(rows),
+               C.byref(blocks))
+        assert rows.value == tile, T
+        assert blocks.value == I // (64 if tile == 16 else 128)
