@@ -140,8 +140,7 @@ SIGNATURES = {
     "aima_moe_grouped_prefill_logits": (C.c_int, [_LP, _vp, _vp, _i64, _vp, _i32, _f32, _vp,
                                                   _vp, _vp, C.POINTER(PrefillOptionsC), _vp,
                                                   C.c_size_t, _vp]),
-    "aima_moe_prefill_tiling": (C.c_int, [_LP, _i64, _i32, _i32, C.POINTER(_i32),
-                                          C.POINTER(_i32)]),
+    "aima_moe_prefill_tiling": (C.c_int, [_LP, _i64, _i32, _i32] + [C.POINTER(_i32)] * 3),
     "aima_moe_prefill_workspace_views": (C.c_int, [_LP, _i64, _i32, _vp,
                                                    C.POINTER(PrefillViewsC)]),
     "aima_grouped_schedule_workspace_size": (C.c_int, [_i64, _i32, _i32, _szp]),

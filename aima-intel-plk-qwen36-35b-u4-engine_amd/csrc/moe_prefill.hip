@@ -1478,15 +1478,23 @@ static int64_t down_halves(const PrefillDims& d) {
 // Whether the down GEMM keeps a tile's token rows in LDS
 // (grouped_down_kernel): 4 quantization groups of them (what fits, and enough
 // work to load them for: at inter 256 and 384 it measured 5 to 9 % a call
-// slower up to T = 8000), tiles taller than thin ones, and a block and a
-// quarter per CU.  Per call (hidden 2048, inter 512), resident against
-// grouped_gemm_kernel: 94 blocks (60 experts, k = 2, T = 1000) 96.1 against
-// 92.4 us, 281 (T = 3000) 127.1 against 125.0; 337 (256 experts, k = 8,
-// T = 1200) 230 against 236, T = 2048 270 against 283 (skewed 226 either way),
-// T = 3000 314 against 343.
+// slower up to T = 8000), tiles taller than thin ones, and enough blocks to
+// hide one's row loads behind another's columns: a block and a half per CU
+// where it computes 512 of at least 1536 columns.  Below that the other kernel
+// loads a tile's rows for half or all of the columns at once, and the loads
+// only pay in very large calls.  Per call at inter 512, resident against
+// grouped_gemm_kernel: hidden 2048, 60 experts, k = 2, T = 4000 (376 blocks)
+// 146.5 against 139.4 us, k = 8, T = 2048 (576) 200 against 204; 256 experts,
+// k = 8, T = 2048 249 against 259, T = 3000 (844) 292 against 305, skewed 267
+// against 269; hidden 1536, 256 experts, k = 2, T = 12000 (846) 308 against 332,
+// skewed 280 against 276; hidden 1024, k = 2, T = 8192 (384) 179 against 169,
+// k = 8, T = 32768 (4608) 1140 against 1181; hidden 768, k = 8, T = 3000 (422)
+// 164 against 141, T = 16384 (2304) 528 against 502.
 static bool down_rows_resident(const PrefillDims& d) {
   const int64_t splits = (d.H + 8 * kDownChunk - 1) / (8 * kDownChunk);
-  return d.I == 128 * kDownGroups && d.A > 32 * (int64_t)d.E && down_halves(d) * splits >= 320;
+  const int64_t least = d.H >= 1536 ? 384 : 3200;
+  return d.I == 128 * kDownGroups && d.H >= 1024 && d.A > 32 * (int64_t)d.E &&
+         down_halves(d) * splits >= least;
 }
 
 // Its column chunks per block: 8 (one per wave) until 16 still leave six
@@ -1786,8 +1794,9 @@ extern "C" int aima_moe_prefill_workspace_views(const aima_moe_layer* layer, int
 
 extern "C" int aima_moe_prefill_tiling(const aima_moe_layer* layer, int64_t tokens, int32_t k,
                                        int32_t output_mode, int32_t* tile_rows,
-                                       int32_t* gateup_tile_blocks) {
-  AIMA_REQUIRE(layer && tile_rows && gateup_tile_blocks, "moe_prefill_tiling: null pointer");
+                                       int32_t* gateup_tile_blocks, int32_t* down_rows) {
+  AIMA_REQUIRE(layer && tile_rows && gateup_tile_blocks && down_rows,
+               "moe_prefill_tiling: null pointer");
   AIMA_REQUIRE(tokens > 0 && k > 0, "moe_prefill_tiling: tokens and k must be positive");
   AIMA_REQUIRE(output_mode == AIMA_PREFILL_FULL_F16 || output_mode == AIMA_PREFILL_ROUTED_F32,
                "moe_prefill_tiling: unknown output mode");
@@ -1795,6 +1804,7 @@ extern "C" int aima_moe_prefill_tiling(const aima_moe_layer* layer, int64_t toke
       prefill_dims(layer, tokens, k, output_mode != AIMA_PREFILL_ROUTED_F32);
   *tile_rows = 1 << d.bm_log2;
   *gateup_tile_blocks = gateup_blocks(d);
+  *down_rows = d.bm_log2 != kMinTileLog2 && down_rows_resident(d) ? kDownRows : *tile_rows;
   return AIMA_OK;
 }
 

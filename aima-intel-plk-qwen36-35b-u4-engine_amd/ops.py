@@ -691,12 +691,13 @@ def prefill_workspace_views(layer: MoeLayerWeights, tokens: int, k: int, ws: Wor
 
 
 def prefill_tiling(layer: MoeLayerWeights, tokens: int, k: int, with_shared: bool = True):
-    """(rows of a full M tile, gate/up blocks per tile) of a prefill call."""
-    rows, blocks = C.c_int32(), C.c_int32()
+    """(rows of a full M tile, gate/up blocks per tile, rows of a down block) of
+    a prefill call."""
+    rows, blocks, down = C.c_int32(), C.c_int32(), C.c_int32()
     mode = _lib.AIMA_PREFILL_FULL_F16 if with_shared else _lib.AIMA_PREFILL_ROUTED_F32
     call("aima_moe_prefill_tiling", C.byref(layer.c()), int(tokens), int(k), mode, C.byref(rows),
-         C.byref(blocks))
-    return rows.value, blocks.value
+         C.byref(blocks), C.byref(down))
+    return rows.value, blocks.value, down.value
 
 
 def build_grouped_schedule(ids: torch.Tensor, router_weights: torch.Tensor, experts: int,

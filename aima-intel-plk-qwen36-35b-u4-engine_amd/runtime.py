@@ -250,7 +250,7 @@ class GroupedU4PrefillRuntime:
             if capture:
                 run.grouped_swiglu_f32 = capture["swiglu_f32"]
                 run.grouped_contributions_f32 = capture["contributions_f32"]
-            _, blocks = ops.prefill_tiling(layer, T, k, with_shared=inp.include_shared)
+            _, blocks, _ = ops.prefill_tiling(layer, T, k, with_shared=inp.include_shared)
             run.gateup_work_tile_count = int(v["tile_count"].item()) * blocks
             run.active_experts = int((counts > 0).sum().item())
             run.max_group_size = int(counts.max().item())

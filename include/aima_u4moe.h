@@ -473,13 +473,14 @@ int aima_moe_prefill_workspace_views(const aima_moe_layer* layer, int64_t tokens
                                      int32_t k, void* workspace,
                                      aima_prefill_views* views);
 
-/* How a prefill call of these sizes cuts its gate/up GEMM: rows of a full M
- * tile and blocks per tile (the work tiles of a call are tile_count of the
- * views times these; RunLayer's gateup_work_tile_count).  output_mode as in
+/* How a prefill call of these sizes cuts its GEMMs: rows of a full M tile,
+ * gate/up blocks per tile (the work tiles of a call are tile_count of the views
+ * times these; RunLayer's gateup_work_tile_count) and token rows per block of
+ * the down GEMM (128: half a tile, resident in LDS).  output_mode as in
  * aima_prefill_options. */
 int aima_moe_prefill_tiling(const aima_moe_layer* layer, int64_t tokens, int32_t k,
                             int32_t output_mode, int32_t* tile_rows,
-                            int32_t* gateup_blocks);
+                            int32_t* gateup_blocks, int32_t* down_rows);
 
 /* Workspace bytes for aima_grouped_schedule. */
 int aima_grouped_schedule_workspace_size(int64_t tokens, int32_t k,

@@ -295,9 +295,9 @@ def test_prefill_workspace_holds_every_tile(pkg, T, k, E):
     L.call("aima_moe_prefill_workspace_views", C.byref(lc), T, k, C.c_void_p(base), C.byref(v))
     capacity = (v.token_map - v.tiles) // 16
     assert base + size >= v.contributions + (T * k + T) * 2048 * 2
-    rows, blocks = C.c_int32(), C.c_int32()
+    rows, blocks, down = C.c_int32(), C.c_int32(), C.c_int32()
     L.call("aima_moe_prefill_tiling", C.byref(lc), T, k, L.AIMA_PREFILL_FULL_F16, C.byref(rows),
-           C.byref(blocks))
+           C.byref(blocks), C.byref(down))
     assert rows.value in (16, 256) and blocks.value == 512 // (64 if rows.value == 16 else 128)
     rng = np.random.default_rng(T * 31 + k * 7 + E)
     zipf = 1.0 / np.arange(1, E + 1) ** 1.1
@@ -380,10 +380,36 @@ def test_prefill_thin_tile_rule(pkg, H, I, E, k, shared, last):
     them up to 1.7 times slower than 256-row ones."""
     L = pkg._lib
     lc = _fake_layer(pkg, H=H, I=I, E=E)
-    rows, blocks = C.c_int32(), C.c_int32()
+    rows, blocks, down = C.c_int32(), C.c_int32(), C.c_int32()
     for T, tile in ((1, 16), (last, 16), (last + 1, 256), (100000, 256)):
         L.call("aima_moe_prefill_tiling", C.byref(lc), T, k,
                L.AIMA_PREFILL_FULL_F16 if shared else L.AIMA_PREFILL_ROUTED_F32, C.byref(rows),
-               C.byref(blocks))
+               C.byref(blocks), C.byref(down))
         assert rows.value == tile, T
         assert blocks.value == I // (64 if tile == 16 else 128)
+
+
+@pytest.mark.parametrize("H,I,E,k,first", [
+    (2048, 512, 256, 8, 1352),    # 384 blocks of 128 rows x 512 columns
+    (1536, 512, 60, 8, 1807),
+    (2048, 512, 256, 1, 8193),    # 32 assignments per expert
+    (1024, 512, 60, 8, 22742),    # 3200 blocks
+    (768, 512, 256, 8, None),
+    (2048, 384, 256, 8, None),
+])
+def test_prefill_resident_down_rule(pkg, H, I, E, k, first):
+    """The fewest tokens whose down GEMM keeps its token rows in LDS: below,
+    and at narrow hidden sizes, it was up to 16 % slower a call."""
+    L = pkg._lib
+    lc = _fake_layer(pkg, H=H, I=I, E=E)
+    rows, blocks, down = C.c_int32(), C.c_int32(), C.c_int32()
+
+    def down_rows(T):
+        L.call("aima_moe_prefill_tiling", C.byref(lc), T, k, L.AIMA_PREFILL_FULL_F16,
+               C.byref(rows), C.byref(blocks), C.byref(down))
+        return down.value
+
+    if first is None:
+        assert [down_rows(T) for T in (4000, 16384, 100000)] == [256] * 3
+    else:
+        assert down_rows(first - 1) == 256 and down_rows(first) == 128

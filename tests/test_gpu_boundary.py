@@ -201,7 +201,7 @@ def test_run_layer_work_tiles(pkg, dev, layer_c2, T, tile, units):
     run = rt.RunLayer(rt.LoadLayer(layer), pkg.GroupedU4PrefillInput(
         pkg.synth.activations(T, 2048, 95, dev), ids, w.reshape(-1), capture_intermediates=True))
     counts = np.bincount(ids.cpu().numpy().reshape(-1), minlength=256)
-    assert pkg.prefill_tiling(layer, T, 8, with_shared=False) == (tile, 512 // units)
+    assert pkg.prefill_tiling(layer, T, 8, with_shared=False)[:2] == (tile, 512 // units)
     assert run.gateup_work_tile_count == int((-(-counts // tile)).sum()) * (512 // units)
 
 

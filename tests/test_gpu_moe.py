@@ -272,6 +272,17 @@ def test_prefill_largest_batch(pkg, dev, layer_full):
     del out, x
 
 
+def _off_alignment(layer):
+    """Moves scales and zero points one element off their vector alignment."""
+    def off(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.reshape(-1)
+        return flat[1:].reshape(t.shape)
+
+    for w in (layer.gate_up, layer.down, layer.shared_gate_up, layer.shared_down):
+        w.scale, w.zp = off(w.scale), off(w.zp)
+
+
 @pytest.mark.parametrize("H,I", [(512, 512), (512, 128), (768, 384)])
 @pytest.mark.parametrize("experts", [96, 16])
 @pytest.mark.parametrize("shift", [0, 1])
@@ -285,13 +296,7 @@ def test_prefill_thin_tiles(pkg, dev, H, I, experts, shift):
     layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=experts, seed=300 + H + I, device=dev)
     mw = moe_to_oracle(layer)
     if shift:
-        def off(t):
-            flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)
-            flat[1:] = t.reshape(-1)
-            return flat[1:].reshape(t.shape)
-
-        for w in (layer.gate_up, layer.down, layer.shared_gate_up, layer.shared_down):
-            w.scale, w.zp = off(w.scale), off(w.zp)
+        _off_alignment(layer)
     counts = [1, 15, 16, 17, 31, 32, 33] if experts == 96 else [1, 15, 16, 17, 31, 32, 33, 257]
     ids = np.repeat(np.arange(len(counts)) * (experts // len(counts)), counts).astype(np.int32)
     ids = np.random.default_rng(H + I).permutation(ids)[:, None].copy()
@@ -325,15 +330,17 @@ def test_prefill_thin_tiles_unbiased(pkg, dev, H, I):
     assert abs(off) <= 6 * 2.0 ** -11 / np.sqrt(ref.size)
 
 
-@pytest.mark.parametrize("H,reps,more", [(2048, 3, 700), (768, 6, 1300)])
-@pytest.mark.parametrize("capture", [False, True])
-def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture):
+@pytest.mark.parametrize("H,reps,more", [(2048, 4, 700), (2304, 4, 100)])
+@pytest.mark.parametrize("capture,shift", [(False, 0), (False, 1), (True, 0)])
+def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture, shift):
     """The down GEMM that keeps a tile's token rows in LDS (inter 512, over 32
-    assignments per expert, at least 320 blocks): remainders around each 32-row
-    block of both 128-row halves, thin halves, and a column count that leaves
-    waves of a block without a chunk (768).  With the f32 copies requested, the
-    f16 contributions are those values rounded.  Tolerance as the other
-    prefill tests."""
+    assignments per expert, at least 384 blocks at hidden 1536 and more):
+    remainders around each 32-row block of both 128-row halves, thin halves, and
+    a column count that leaves waves of a block without a chunk (2304).  Scales
+    and zero points off their vector alignment (shift) take the instance that
+    loads them value by value.  With the f32 copies requested, the f16
+    contributions are those values rounded.  Tolerance as the other prefill
+    tests."""
     I = 512
     counts = [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 256, 289] * reps + [more]
     layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=len(counts), seed=400 + H, device=dev)
@@ -341,7 +348,9 @@ def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture):
     ids = np.repeat(np.arange(len(counts)), counts).astype(np.int32)
     ids = np.random.default_rng(H + I).permutation(ids)[:, None].copy()
     T = len(ids)
-    assert T > 32 * len(counts) and -(-2 * T // 128) * -(-H // 512) >= 320
+    assert T > 32 * len(counts) and -(-2 * T // 128) * -(-H // 512) >= 384
+    if shift:
+        _off_alignment(layer)
     x = pkg.synth.activations(T, H, 401, dev)
     w = torch.rand((T, 1), device=dev) + 0.5
     d_ids = torch.from_numpy(ids).to(dev)
