@@ -57,13 +57,15 @@ __device__ __forceinline__ void rg_read(const uint16_t* row, int swz, int k0, fl
 // selection, against 57 to 61 here; 64 x 64 tiles with two K halves, read the
 // same way, took 68 us at T = 2048 where this takes 28 (f16 input).
 // Blocks are mapped XCD-aware: a token tile's expert blocks run on one XCD.
+// The grid is 8 token tiles x the expert tiles, by the rest of the token tiles:
+// in one dimension 2^24 tokens of 1024 experts would pass 2^32 threads.
 //
 // Rows past T (tokens) or E (experts) load the last row (valid memory) and
 // are never stored; k past H load as zeros.  H % 16 == 0 and both matrices
 // 16-byte aligned (checked on the host).
 template <typename X, int NA>
 __global__ __launch_bounds__(kRgThreads, 2) void router_gemm_kernel(
-    const X* __restrict__ x, const float* __restrict__ w, int64_t T, int E, int H, int ey,
+    const X* __restrict__ x, const float* __restrict__ w, int64_t T, int E, int H,
     float* __restrict__ logits) {
   constexpr int kXVals = 16 / sizeof(X);         // values of a 16-byte piece
   constexpr int kXPieces = kRgChunk / kXVals;    // pieces of a token row's step
@@ -74,9 +76,9 @@ __global__ __launch_bounds__(kRgThreads, 2) void router_gemm_kernel(
   constexpr int kSmem = 2 * (kXBytes + kWBytes) > kPartBytes ? 2 * (kXBytes + kWBytes) : kPartBytes;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kSmem];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int p = blockIdx.x, slot = p >> 3;
-  const int64_t t0 = (int64_t)((slot / ey) * 8 + (p & 7)) * (32 * NA);
-  const int e0 = (slot % ey) * 32;
+  const int p = blockIdx.x;
+  const int64_t t0 = ((int64_t)blockIdx.y * 8 + (p & 7)) * (32 * NA);
+  const int e0 = (p >> 3) * 32;
   if (t0 >= T) return;
 
   const X* xp[kXPer];
@@ -192,11 +194,13 @@ int router_gemm_launch(const X* x, int64_t tokens, int experts, int64_t hidden, 
   const int ey = (experts + 31) / 32;
   const int64_t wide = (tokens + 63) / 64, narrow = (tokens + 31) / 32;
   if (wide * ey > 256) {
-    hipLaunchKernelGGL((router_gemm_kernel<X, 2>), dim3((unsigned)(round_up(wide, 8) * ey)),
-                       dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, ey, logits);
+    hipLaunchKernelGGL((router_gemm_kernel<X, 2>),
+                       dim3((unsigned)(8 * ey), (unsigned)(round_up(wide, 8) / 8)),
+                       dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, logits);
   } else {
-    hipLaunchKernelGGL((router_gemm_kernel<X, 1>), dim3((unsigned)(round_up(narrow, 8) * ey)),
-                       dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, ey, logits);
+    hipLaunchKernelGGL((router_gemm_kernel<X, 1>),
+                       dim3((unsigned)(8 * ey), (unsigned)(round_up(narrow, 8) / 8)),
+                       dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, logits);
   }
   return launch_check("router_gemm");
 }

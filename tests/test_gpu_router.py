@@ -60,6 +60,24 @@ def test_router_gemm_edges(pkg, dev, T, E, H, f32):
     assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")
 
 
+def test_router_gemm_most_tokens(pkg, dev):
+    """The most tokens and experts of one call (2^24 x 1024): more than 2^32
+    threads.  4096 rows repeated: every logit of the first and of the last
+    4096."""
+    if torch.cuda.mem_get_info()[0] < 130 << 30:
+        pytest.skip("needs 100 GB of device memory")
+    T, H, E = 1 << 24, 256, 1024
+    x = pkg.synth.activations(4096, H, 90, dev)
+    W = _router(E, H, 91, dev)
+    _, _, logits = pkg.router_gemm_topk(x.repeat(T // 4096, 1), W, 1)
+    ref = x.double() @ W.double().T
+    bound = (x.double().abs() @ W.double().abs().T) * H * 2.0 ** -24
+    assert bool(((logits[:4096].double() - ref).abs() <= bound).all())
+    assert torch.equal(logits[-4096:], logits[:4096])
+    del logits
+    torch.cuda.empty_cache()
+
+
 def test_router_gemm_f16_input(pkg, dev):
     """An f16 input is widened exactly: the same logits as its f32 copy."""
     T, H, E = 129, 2048, 256
