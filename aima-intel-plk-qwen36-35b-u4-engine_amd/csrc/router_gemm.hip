@@ -54,7 +54,7 @@ __device__ __forceinline__ void rg_read(const uint16_t* row, int swz, int k0, fl
 // H = 2048).  The output has only 512 32 x 32 tiles there, two per CU: K split
 // over the waves of a block fills the chip.  Rows read straight into the
 // operands' lanes (32 rows per load) made T = 4096 f32 88 us a call with its
-// selection, against 57 to 61 here; 64 x 64 tiles with two K halves, read the
+// selection, against 55 here; 64 x 64 tiles with two K halves, read the
 // same way, took 68 us at T = 2048 where this takes 28 (f16 input).
 // Blocks are mapped XCD-aware: a token tile's expert blocks run on one XCD.
 // The grid is 8 token tiles x the expert tiles, by the rest of the token tiles:
@@ -184,17 +184,20 @@ __global__ __launch_bounds__(kRgThreads, 2) void router_gemm_kernel(
   }
 }
 
-// 64 tokens per block (fewer reads of the router's rows) once that leaves
-// more than one block per CU: T = 2048, E = 256 (256 such blocks) 35.3 us a
-// call against 33.3 in 512 blocks of 32 tokens; T = 4096, f16: 52.6 against
-// 55.5 (f32: 61.4 against 56.8).
+// 64 tokens per block (fewer reads of the router's rows) for f16 tokens, once
+// that leaves more than one block per CU: T = 2048, E = 256 (256 such blocks)
+// 35.3 us a call against 33.3 in 512 blocks of 32 tokens; T = 4096 52.6 against
+// 55.5.  With f32 tokens such a block takes 96 KB of LDS, one per CU instead of
+// two: T = 2500, E = 256 58.0 against 43.2, T = 4096 59.8 against 54.9, T =
+// 16384 222 against 197.
 template <typename X>
 int router_gemm_launch(const X* x, int64_t tokens, int experts, int64_t hidden, const float* w,
                        float* logits, hipStream_t st) {
+  constexpr bool kWide = sizeof(X) == 2;
   const int ey = (experts + 31) / 32;
   const int64_t wide = (tokens + 63) / 64, narrow = (tokens + 31) / 32;
-  if (wide * ey > 256) {
-    hipLaunchKernelGGL((router_gemm_kernel<X, 2>),
+  if (kWide && wide * ey > 256) {
+    hipLaunchKernelGGL((router_gemm_kernel<X, kWide ? 2 : 1>),
                        dim3((unsigned)(8 * ey), (unsigned)(round_up(wide, 8) / 8)),
                        dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, logits);
   } else {

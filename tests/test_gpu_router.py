@@ -39,14 +39,16 @@ def test_router_gemm_topk(pkg, dev, T, E, k, H):
     assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")
 
 
-@pytest.mark.parametrize("T,E,H", [(31, 33, 16), (33, 32, 144), (65, 64, 384),
-                                   (16449, 17, 272)])
+@pytest.mark.parametrize("T,E,H", [(31, 33, 16), (33, 32, 144), (65, 64, 384), (300, 100, 400),
+                                   (16449, 17, 272), (16449, 130, 272)])
 @pytest.mark.parametrize("f32", [True, False])
 def test_router_gemm_edges(pkg, dev, T, E, H, f32):
-    """Both block widths (16,449 tokens: 64-token blocks), partial blocks in
-    both dimensions, K below one 128-wide step, with a partial last step and
-    with an odd number of steps.  f32 sums of H products: each at most
-    H * 2^-24 of the sum of its terms' magnitudes off."""
+    """Both block widths (f16, 16,449 tokens: 64-token blocks, of one and of
+    several expert columns), partial blocks in both dimensions, K below one
+    128-wide step, with a partial last step and with an odd number of steps.
+    f32 sums of H products: each at most H * 2^-24 of the sum of its terms'
+    magnitudes off.  An f16 input is widened exactly: the same logits as its
+    f32 copy, whatever blocks either takes."""
     x = pkg.synth.activations(T, H, T + H, dev)
     x = x.float() if f32 else x
     W = _router(E, H, T + 2, dev)
@@ -55,6 +57,8 @@ def test_router_gemm_edges(pkg, dev, T, E, H, f32):
     ref = x.double() @ W.double().T
     bound = (x.double().abs() @ W.double().abs().T) * H * 2.0 ** -24
     assert bool(((logits.double() - ref).abs() <= bound).all())
+    if not f32:
+        assert torch.equal(logits, pkg.router_gemm_topk(x.float(), W, 4)[2])
     ref_ids, ref_w = oracle.router_topk_tokens(logits.cpu().numpy(), 4)
     assert np.array_equal(ids.cpu().numpy(), ref_ids)
     assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")
