@@ -184,6 +184,76 @@ __global__ __launch_bounds__(kRgThreads, 2) void router_gemm_kernel(
   }
 }
 
+// Short rows (rows_short): a block of 8 waves owns 64 tokens x 64 experts; wave
+// w computes the 32 x 32 quarter w % 4 over the K half w / 4, and the two halves
+// are added through LDS (half 0 + half 1, the same order every call).  Each lane
+// loads 4 consecutive k of its token row and of its expert row per 8 k straight
+// into the operands.
+//
+// Bound: the logits' bytes.  There are too few k to split over eight waves, and
+// a block of the kernel above holds 64 KB or more of LDS whatever they are, so
+// that one or two per CU wait for their few loads.
+constexpr int kRgShortTile = 64;
+
+__device__ __forceinline__ float4 rg_load4(const float* p) {
+  return *reinterpret_cast<const float4*>(p);
+}
+__device__ __forceinline__ float4 rg_load4(const uint16_t* p) {
+  const u32x2 d = *reinterpret_cast<const u32x2*>(p);
+  const uint32_t a = d[0], b = d[1];
+  return make_float4(h2f((uint16_t)(a & 0xffffu)), h2f((uint16_t)(a >> 16)),
+                     h2f((uint16_t)(b & 0xffffu)), h2f((uint16_t)(b >> 16)));
+}
+
+template <typename X>
+__global__ __launch_bounds__(kRgThreads) void router_gemm_short_kernel(
+    const X* __restrict__ x, const float* __restrict__ w, int64_t T, int E, int H,
+    float* __restrict__ logits) {
+  __shared__ float part[4][16][64];  // K-half 1 partial sums, [quarter][acc][lane]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int q = wave & 3, kh = wave >> 2;
+  const int64_t t0 = (int64_t)blockIdx.x * kRgShortTile + 32 * (q >> 1);
+  const int e0 = (int)blockIdx.y * kRgShortTile + 32 * (q & 1);
+  const int64_t tr = t0 + (lane & 31) < T ? t0 + (lane & 31) : T - 1;
+  const int er = e0 + (lane & 31) < E ? e0 + (lane & 31) : E - 1;
+  const int half = H / 2;
+  const X* xp = x + tr * H + kh * half + 4 * (lane >> 5);
+  const float* wp = w + (int64_t)er * H + kh * half + 4 * (lane >> 5);
+  f32x16_t acc = f32x16_t{};
+  for (int k = 0; k < half; k += 8) {
+    const float4 a = rg_load4(xp + k), b = rg_load4(wp + k);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+  }
+  if (kh == 1) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part[q][i][lane] = acc[i];
+  }
+  __syncthreads();
+  if (kh == 1) return;
+  const int e = e0 + (lane & 31);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int64_t t = t0 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    const float v = acc[i] + part[q][i][lane];
+    if (t < T && e < E) logits[t * E + e] = v;
+  }
+}
+
+// Where short rows pay, direct against through LDS, us a call with its
+// selection: hidden 128, f16, E = 512, T = 16384 73 against 97, f32 73 against
+// 107; hidden 192 85 against 97, f32 85 against 107; hidden 256, f16 97 against
+// 97, E = 64, T = 8192 19 against 16, f32 100 against 105 and 20 against 19.
+// In the largest calls that goes on to hidden 384 for f32 rows, which take more
+// LDS: E = 1024, T = 16384 248 against 272 (f16 236 against 237), T = 65536 1012
+// against 1085 (f16 945 against 925); hidden 512, E = 512 84 against 77.  One
+// rule for both types: an f16 input has the bits of its f32 copy.
+bool rows_short(int64_t tokens, int experts, int64_t hidden) {
+  return hidden <= (tokens * experts >= (1 << 23) ? 384 : 192);
+}
+
 // 64 tokens per block (fewer reads of the router's rows) for f16 tokens, once
 // that leaves more than one block per CU: T = 2048, E = 256 (256 such blocks)
 // 35.3 us a call against 33.3 in 512 blocks of 32 tokens; T = 4096 52.6 against
@@ -196,7 +266,12 @@ int router_gemm_launch(const X* x, int64_t tokens, int experts, int64_t hidden, 
   constexpr bool kWide = sizeof(X) == 2;
   const int ey = (experts + 31) / 32;
   const int64_t wide = (tokens + 63) / 64, narrow = (tokens + 31) / 32;
-  if (kWide && wide * ey > 256) {
+  if (rows_short(tokens, experts, hidden)) {
+    const dim3 grid((unsigned)((tokens + kRgShortTile - 1) / kRgShortTile),
+                    (unsigned)((experts + kRgShortTile - 1) / kRgShortTile));
+    hipLaunchKernelGGL(router_gemm_short_kernel<X>, grid, dim3(kRgThreads), 0, st, x, w, tokens,
+                       experts, (int)hidden, logits);
+  } else if (kWide && wide * ey > 256) {
     hipLaunchKernelGGL((router_gemm_kernel<X, kWide ? 2 : 1>),
                        dim3((unsigned)(8 * ey), (unsigned)(round_up(wide, 8) / 8)),
                        dim3(kRgThreads), 0, st, x, w, tokens, experts, (int)hidden, logits);

@@ -39,16 +39,17 @@ def test_router_gemm_topk(pkg, dev, T, E, k, H):
     assert_parity(w.cpu().numpy(), ref_w, tol=1e-6, what="router weights")
 
 
-@pytest.mark.parametrize("T,E,H", [(31, 33, 16), (33, 32, 144), (65, 64, 384), (300, 100, 400),
-                                   (16449, 17, 272), (16449, 130, 272)])
+@pytest.mark.parametrize("T,E,H", [(31, 33, 16), (33, 32, 144), (129, 65, 192), (65, 64, 208),
+                                   (65, 64, 384), (300, 100, 400), (16449, 17, 272),
+                                   (16449, 130, 272), (16449, 514, 272)])
 @pytest.mark.parametrize("f32", [True, False])
 def test_router_gemm_edges(pkg, dev, T, E, H, f32):
-    """Both block widths (f16, 16,449 tokens: 64-token blocks, of one and of
-    several expert columns), partial blocks in both dimensions, K below one
-    128-wide step, with a partial last step and with an odd number of steps.
-    f32 sums of H products: each at most H * 2^-24 of the sum of its terms'
-    magnitudes off.  An f16 input is widened exactly: the same logits as its
-    f32 copy, whatever blocks either takes."""
+    """Short rows (up to 192, in large calls 384) and longer ones, both block
+    widths (f16, 16,449 tokens: 64-token blocks, of one and of several expert
+    columns), partial blocks in both dimensions, partial last steps of K and an
+    odd number of them.  f32 sums of H products: each at most H * 2^-24 of the
+    sum of its terms' magnitudes off.  An f16 input is widened exactly: the same
+    logits as its f32 copy, whatever blocks either takes."""
     x = pkg.synth.activations(T, H, T + H, dev)
     x = x.float() if f32 else x
     W = _router(E, H, T + 2, dev)
@@ -68,9 +69,9 @@ def test_router_gemm_most_tokens(pkg, dev):
     """The most tokens and experts of one call (2^24 x 1024): more than 2^32
     threads.  4096 rows repeated: every logit of the first and of the last
     4096."""
-    if torch.cuda.mem_get_info()[0] < 130 << 30:
-        pytest.skip("needs 100 GB of device memory")
-    T, H, E = 1 << 24, 256, 1024
+    if torch.cuda.mem_get_info()[0] < 150 << 30:
+        pytest.skip("needs 120 GB of device memory")
+    T, H, E = 1 << 24, 400, 1024
     x = pkg.synth.activations(4096, H, 90, dev)
     W = _router(E, H, 91, dev)
     _, _, logits = pkg.router_gemm_topk(x.repeat(T // 4096, 1), W, 1)
