@@ -250,7 +250,7 @@ int rmsnorm_launch(const uint16_t* x, const float* weight, int64_t rows, int64_t
 constexpr int kRouterMaxPerLane = 16;  // experts <= 1024
 
 // PER = logits per lane (experts <= 64 PER); lane r keeps the rank-r pick in
-// registers, and lane 0 sums the picks in rank order through shuffles.
+// registers, and every lane sums the picks in rank order as they are found.
 template <int PER>
 __global__ __launch_bounds__(256) void router_topk_kernel(
     const float* __restrict__ logits, int64_t tokens, int experts, int k,
