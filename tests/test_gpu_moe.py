@@ -371,6 +371,36 @@ def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture, shift):
     assert_parity(got, ref, what=f"resident down rows H={H} I={I}")
 
 
+@pytest.mark.parametrize("H,I", [(512, 256), (768, 384)])
+def test_prefill_capture_tall_tiles(pkg, dev, H, I):
+    """The f32 copies of tiles over 32 rows (every height in 32-row blocks, full
+    tiles, remainders) where the down GEMM does not keep its token rows: near
+    the oracle's, and the f16 rows are those values rounded, bit for bit."""
+    counts = [33, 64, 65, 97, 130, 161, 200, 256, 290]
+    layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=len(counts), seed=450 + H, device=dev)
+    mw = moe_to_oracle(layer)
+    ids = np.repeat(np.arange(len(counts)), counts).astype(np.int32)
+    ids = np.random.default_rng(H).permutation(ids)[:, None].copy()
+    T = len(ids)
+    assert pkg.prefill_tiling(layer, T, 1, with_shared=False)[::2] == (256, 256)
+    x = pkg.synth.activations(T, H, 451, dev)
+    w = torch.rand((T, 1), device=dev) + 0.5
+    ws, cap = pkg.Workspace(dev), {}
+    pkg.grouped_moe_prefill_routed(layer, x, torch.from_numpy(ids).to(dev), w,
+                                   expert_used_count=1, ws=ws, capture_f32=cap)
+    rows = pkg.prefill_workspace_views(layer, T, 1, ws, with_shared=False)
+    assert torch.equal(rows["swiglu"], cap["swiglu_f32"].half())
+    assert torch.equal(rows["contributions"], cap["contributions_f32"].half())
+    token = rows["token_map"].long().cpu()
+    ref = oracle.moe_routed_tokens(mw, f16_to_f32(x), ids, w.cpu().numpy(), threads=THREADS)
+    assert_parity(cap["contributions_f32"].cpu().numpy(), ref[token.numpy()], what="contributions")
+    for row in range(0, T, 97):
+        t = int(token[row])
+        d = oracle.moe_ffn_token_detail(mw, f16_to_f32(x[t]), None, ids[t], w[t].cpu().numpy())
+        assert_parity(cap["swiglu_f32"][row].cpu().numpy(), d["selected_swiglu"].reshape(-1),
+                      what=f"swiglu row {row}")
+
+
 @pytest.mark.parametrize("T,E,k", [(128, 256, 8), (1025, 8, 1), (147, 1024, 7), (32768, 256, 8),
                                    (32770, 130, 8)])
 def test_schedule_launch_forms(pkg, dev, T, E, k):
