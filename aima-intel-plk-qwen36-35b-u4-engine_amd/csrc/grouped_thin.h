@@ -16,7 +16,7 @@
 // codes alone as (subnormal) operands, takes two instructions less a word, but
 // an infinite x makes it inf - inf, sum(x) takes MFMAs of its own, and its
 // extra fold and registers cost more than they save: T = 777 (24 rows an
-// expert) 168 us a call against 157 here, T = 96 110.5 against 110.3.
+// expert) 167 us a call against 151 here, T = 96 109.5 against 107.4.
 //
 // A block of NW waves owns one tile and 32 NW weight rows (gate/up: 16 NW
 // gate and the matching 16 NW up rows).  v_mfma_f32_16x16x32_f16: the tokens
@@ -24,7 +24,7 @@
 // quarter l / 16 of the group: one 16-byte load per row and group), so a
 // lane's results all belong to its own weight row, whose scale and zero point
 // it loads itself.  Each wave runs 2 x 16 weight rows against NB x 16 tokens.
-// Tokens reach LDS through registers, CH groups at a time in two buffers,
+// Tokens reach LDS through registers, 4 groups at a time in two buffers,
 // already in the operands' order (low nibbles' k, then high nibbles' k of
 // each 16), with 16-byte piece p of row r in slot p ^ (r & 15) of its 256
 // bytes: no bank conflicts.  The next 4 groups of weights are in flight while
@@ -45,11 +45,11 @@ namespace aima {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThinThreads = 256;
-constexpr int kThinTurn = 4;  // groups per turn of the weight registers
+constexpr int kThinTurn = 4;  // groups per turn of the weight registers and token buffers
 
-__host__ __device__ constexpr int thin_buf_bytes(int nb, int ch) { return nb * 16 * ch * 256; }
-inline size_t thin_lds_bytes(int nb, int ch, int64_t GK) {
-  return (size_t)(GK > ch ? 2 : 1) * thin_buf_bytes(nb, ch);
+__host__ __device__ constexpr int thin_buf_bytes(int nb) { return nb * 16 * kThinTurn * 256; }
+inline size_t thin_lds_bytes(int nb, int64_t GK) {
+  return (size_t)(GK > kThinTurn ? 2 : 1) * thin_buf_bytes(nb);
 }
 
 struct ThinArgs {
@@ -156,10 +156,9 @@ __device__ __forceinline__ float as_f32_value(float v) {
   return v;
 }
 
-template <bool GATEUP, int NB, int CH, bool V4, bool CAP, int TH>
+template <bool GATEUP, int NB, bool V4, bool CAP, int TH>
 __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_layer& L, uint8_t* smem,
                                           int e, int64_t row0, int rows, int ntile) {
-  static_assert(kThinTurn % CH == 0 && CH % 2 == 0, "whole token chunks per turn");
   constexpr int WD = kThinTurn, NW = TH / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15, q = lane >> 4;
@@ -168,7 +167,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
   const int GK = (int)(K >> 7);
   const bool routed = e < L.experts;
   const int64_t eoff = routed ? e : 0;
-  constexpr int kBuf = thin_buf_bytes(NB, CH);
+  constexpr int kBuf = thin_buf_bytes(NB);
 
   // this lane's two weight rows: gate and up row of unit ntile * 64 +
   // wave * 16 + n, or output columns ntile * 128 + wave * 32 + n and + 16
@@ -205,8 +204,8 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
     d[1] = gload16(wp[1] + gc * 64);
   };
 
-  // token rows staged by this thread: rows tid / (8 CH) + ..., 32 bytes each
-  constexpr int kPairs = CH * 8;                 // 32-byte pieces of a row per chunk
+  // token rows staged by this thread: rows tid / (8 WD) + ..., 32 bytes each
+  constexpr int kPairs = WD * 8;                 // 32-byte pieces of a row per turn
   constexpr int kPer = NB * 16 * kPairs / TH;
   constexpr int kRowStep = TH / kPairs;
   const int tp = tid % kPairs, trow = tid / kPairs;
@@ -220,10 +219,10 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
   }
   const char* src = reinterpret_cast<const char*>(a.src);
   u32x4 tk[kPer][2];
-  auto load_tokens = [&](int c) {
-    // groups past K (a last, partial chunk) reload the chunk's first group
-    const int g = c * CH + tp / 8;
-    const uint32_t off = (uint32_t)(g < GK ? c * CH * 256 + tp * 32 : c * CH * 256 + (tp & 7) * 32);
+  auto load_tokens = [&](int t) {
+    // groups past K (a last, partial turn) reload the turn's first group
+    const int g = t * WD + tp / 8;
+    const uint32_t off = (uint32_t)(t * WD * 256 + (g < GK ? tp * 32 : (tp & 7) * 32));
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       tk[i][0] = *reinterpret_cast<const u32x4*>(src + soff[i] + off);
@@ -289,49 +288,33 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& a, const aima_moe_laye
     }
   };
 
-  // The tokens of the next chunk are loaded while this one is used and stored
-  // behind it.  Every turn but the last is straight-line code: a branch
+  // The tokens of the next turn are loaded while this one's are used and stored
+  // behind them.  Every turn but the last is straight-line code: a branch
   // around a load would make the compiler wait for the loads before it.
   const int turns = (GK + WD - 1) / WD;
   int g0 = 0;
   for (int t = 0; t + 1 < turns; ++t, g0 += WD) {
     sn[0].load(sp[0], zp[0], zat[0], g0 + WD, GK);
     sn[1].load(sp[1], zp[1], zat[1], g0 + WD, GK);
+    load_tokens(t + 1);
+    const uint8_t* buf = smem + (t & 1) * kBuf;
 #pragma unroll
-    for (int u = 0; u < WD; u += CH) {
-      const int c = (g0 + u) / CH;
-      load_tokens(c + 1);
-      const uint8_t* buf = smem + (c & 1) * kBuf;
-#pragma unroll
-      for (int gi = 0; gi < CH; gi += 2) {
-        group(buf + gi * NB * 16 * 256, w[u + gi], u + gi);
-        group(buf + (gi + 1) * NB * 16 * 256, w[u + gi + 1], u + gi + 1);
-        // two groups are one 128-byte line of a row: asked for together
-        load_w(g0 + u + gi + WD, w[u + gi]);
-        load_w(g0 + u + gi + WD + 1, w[u + gi + 1]);
-      }
-      store_tokens(smem + ((c + 1) & 1) * kBuf);
-      __syncthreads();
+    for (int gi = 0; gi < WD; gi += 2) {
+      group(buf + gi * NB * 16 * 256, w[gi], gi);
+      group(buf + (gi + 1) * NB * 16 * 256, w[gi + 1], gi + 1);
+      // two groups are one 128-byte line of a row: asked for together
+      load_w(g0 + gi + WD, w[gi]);
+      load_w(g0 + gi + WD + 1, w[gi + 1]);
     }
+    store_tokens(smem + ((t + 1) & 1) * kBuf);
+    __syncthreads();
     sz[0] = sn[0];
     sz[1] = sn[1];
   }
+  const uint8_t* last = smem + ((turns - 1) & 1) * kBuf;
 #pragma unroll
-  for (int u = 0; u < WD; u += CH) {
-    if (g0 + u < GK) {
-      const int c = (g0 + u) / CH;
-      const bool more = u + CH < WD && g0 + u + CH < GK;
-      if (more) load_tokens(c + 1);
-      const uint8_t* buf = smem + (c & 1) * kBuf;
-#pragma unroll
-      for (int gi = 0; gi < CH; ++gi) {
-        if (g0 + u + gi < GK) group(buf + gi * NB * 16 * 256, w[u + gi], u + gi);
-      }
-      if (more) {
-        store_tokens(smem + ((c + 1) & 1) * kBuf);
-        __syncthreads();
-      }
-    }
+  for (int gi = 0; gi < WD; ++gi) {
+    if (g0 + gi < GK) group(last + gi * NB * 16 * 256, w[gi], gi);
   }
 
   // lane (n, q): weight rows n (of each 16) and token rows 16 b + 4 q + j.
@@ -388,9 +371,9 @@ __global__ __launch_bounds__(kThinThreads, V4 ? 3 : 2) void grouped_thin_kernel(
   const int slot = p >> 3;
   const int mt = (slot / a.ntiles_n) * 8 + (p & 7);
   if (mt >= *a.tile_count) return;
-  thin_tile<GATEUP, 1, kThinTurn, V4, CAP, kThinThreads>(a, L, thin_smem, a.tiles[4 * mt + 0],
-                                                    a.tiles[4 * mt + 1], a.tiles[4 * mt + 2],
-                                                    slot % a.ntiles_n);
+  thin_tile<GATEUP, 1, V4, CAP, kThinThreads>(a, L, thin_smem, a.tiles[4 * mt + 0],
+                                              a.tiles[4 * mt + 1], a.tiles[4 * mt + 2],
+                                              slot % a.ntiles_n);
 }
 
 }  // namespace aima

@@ -870,7 +870,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
 
   // Tiles of one 32-row block: their time is the dequantization of weights
   // that feed a single MFMA each, so they take the integer operands of
-  // thin_tile.  T = 777, uniform routing: 157 us per call (f16 operands on this
+  // thin_tile.  T = 777, uniform routing: 151 us per call (f16 operands on this
   // block's own path, with one schedule launch more: 182).
   if (tiles[4 * mt + 2] <= 32) {
     const ThinArgs a{src, tiles, tile_count, token_map, row_weight, A, ntiles_n,
@@ -878,9 +878,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
     const int e = tiles[4 * mt + 0], rows = tiles[4 * mt + 2];
     const int64_t row0 = tiles[4 * mt + 1];
     if (rows <= 16) {
-      thin_tile<GATEUP, 1, kThinTurn, V4, CAP, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
+      thin_tile<GATEUP, 1, V4, CAP, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
     } else {
-      thin_tile<GATEUP, 2, kThinTurn, V4, CAP, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
+      thin_tile<GATEUP, 2, V4, CAP, kGemmThreads>(a, L, smem, e, row0, rows, slot % ntiles_n);
     }
     return;
   }
@@ -1175,9 +1175,9 @@ __global__ __launch_bounds__(512, 2) void grouped_down_kernel(
     for (int nt = c0 / 4; nt < c1 / 4; ++nt) {  // 256 columns each
       if (nt > c0 / 4) __syncthreads();
       if (t.rows <= 16) {
-        thin_tile<false, 1, kThinTurn, V4, CAP, 512>(a, L, smem, t.e, t.row0, t.rows, nt);
+        thin_tile<false, 1, V4, CAP, 512>(a, L, smem, t.e, t.row0, t.rows, nt);
       } else {
-        thin_tile<false, 2, kThinTurn, V4, CAP, 512>(a, L, smem, t.e, t.row0, t.rows, nt);
+        thin_tile<false, 2, V4, CAP, 512>(a, L, smem, t.e, t.row0, t.rows, nt);
       }
     }
     return;
@@ -1535,7 +1535,7 @@ static int launch_gemm(const aima_moe_layer& L, const uint16_t* src, const Prefi
                             grouped_thin_kernel<GATEUP, false, false>,
                             grouped_thin_kernel<GATEUP, false, true>),
                        dim3(mtiles * nt), dim3(kThinThreads),
-                       thin_lds_bytes(1, kThinTurn, K / 128), st, L, a);
+                       thin_lds_bytes(1, K / 128), st, L, a);
   } else if (!GATEUP && down_rows_resident(d)) {
     const int chunks = d.H / kDownChunk;
     const int cpb = down_chunks(d);
