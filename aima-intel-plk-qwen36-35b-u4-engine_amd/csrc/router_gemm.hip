@@ -283,28 +283,24 @@ int router_gemm_launch(const X* x, int64_t tokens, int experts, int64_t hidden, 
   return launch_check("router_gemm");
 }
 
-size_t router_ws_bytes(int64_t tokens, int64_t hidden, int input_f32) {
-  return input_f32 ? 0 : kWsHeader + round_up((size_t)tokens * hidden * 4, 256);
-}
-
 }  // namespace
 }  // namespace aima
 
 using namespace aima;
 
-extern "C" int aima_router_gemm_workspace_size(int64_t tokens, int64_t hidden, int32_t input_f32,
-                                               size_t* bytes) {
+extern "C" int aima_router_gemm_workspace_size(int64_t tokens, int64_t hidden,
+                                               int32_t /*input_f32*/, size_t* bytes) {
   AIMA_REQUIRE(bytes, "router_gemm_workspace_size: null pointer");
   AIMA_REQUIRE(tokens > 0 && hidden > 0, "router_gemm_workspace_size: sizes must be positive");
-  *bytes = router_ws_bytes(tokens, hidden, input_f32);
+  *bytes = 0;  // an f16 input is widened in registers
   return AIMA_OK;
 }
 
 extern "C" int aima_router_gemm_topk(const void* hidden_states, int32_t input_f32, int64_t tokens,
                                      int64_t hidden, const float* router_weight, int32_t experts,
                                      int32_t k, float min_weight_sum, float* logits, int32_t* ids,
-                                     float* weights, void* workspace, size_t workspace_bytes,
-                                     void* stream) {
+                                     float* weights, void* /*workspace*/,
+                                     size_t /*workspace_bytes*/, void* stream) {
   AIMA_REQUIRE(hidden_states && router_weight && logits && ids && weights,
                "router_gemm_topk: null pointer");
   AIMA_REQUIRE(tokens > 0 && hidden > 0 && tokens <= (1 << 24) && hidden <= (1 << 20),
@@ -317,10 +313,6 @@ extern "C" int aima_router_gemm_topk(const void* hidden_states, int32_t input_f3
                "router_gemm_topk: k must be in [1, min(16, experts)]");
   AIMA_REQUIRE(min_weight_sum > 0.f, "router_gemm_topk: minimum weight sum must be positive");
   const hipStream_t st = (hipStream_t)stream;
-  // (an f16 input was once widened there; the size a caller queries stays)
-  AIMA_REQUIRE(input_f32 || (workspace && aligned(workspace, 256) &&
-                             workspace_bytes >= router_ws_bytes(tokens, hidden, 0)),
-               "router_gemm_topk: an f16 input needs the workspace");
   const int rc = input_f32 ? router_gemm_launch(static_cast<const float*>(hidden_states), tokens,
                                                 experts, hidden, router_weight, logits, st)
                            : router_gemm_launch(static_cast<const uint16_t*>(hidden_states), tokens,

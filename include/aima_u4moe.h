@@ -174,7 +174,7 @@ int aima_router_fc_topk(const uint16_t* h, const aima_u4_tensor* router,
                         int32_t k, float min_weight_sum, float* logits,
                         int32_t* ids, float* weights, void* stream);
 
-/* Workspace bytes for aima_router_gemm_topk (0 for an f32 input). */
+/* Workspace bytes for aima_router_gemm_topk: 0. */
 int aima_router_gemm_workspace_size(int64_t tokens, int64_t hidden,
                                     int32_t input_f32, size_t* bytes);
 
@@ -184,8 +184,8 @@ int aima_router_gemm_workspace_size(int64_t tokens, int64_t hidden,
  * hidden_states[T][H] . router_weight[E][H]^T in f32 (f32 matrix-core
  * GEMM on `stream`), then the selection of aima_router_topk per token:
  * ids[T][k], weights[T][k] (normalized).  hidden_states is f32
- * (input_f32 = 1) or f16 (0: widened in registers; the workspace of
- * aima_router_gemm_workspace_size is required all the same).
+ * (input_f32 = 1) or f16 (0: widened in registers); workspace is not used
+ * and may be NULL.
  * hidden % 16 == 0, hidden_states and router_weight 16-byte aligned,
  * experts <= 1024, k <= 16. */
 int aima_router_gemm_topk(const void* hidden_states, int32_t input_f32,

@@ -363,6 +363,8 @@ def test_router_gemm_validation(pkg):
     args = lambda x, H: (x, 1, 64, H, p, 256, 8, C.c_float(6.1e-5), p, p, p, None, 0, None)
     assert lib.aima_router_gemm_topk(*args(p, 2040)) == L.AIMA_E_INVALID
     assert lib.aima_router_gemm_topk(*args(odd, 2048)) == L.AIMA_E_INVALID
+    for f32 in (0, 1):  # no pass of its own for either input type
+        assert L.size_query("aima_router_gemm_workspace_size", 8192, 2048, f32) == 0
 
 
 @pytest.mark.parametrize("H,I,E,k,shared,last", [

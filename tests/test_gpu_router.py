@@ -69,8 +69,8 @@ def test_router_gemm_most_tokens(pkg, dev):
     """The most tokens and experts of one call (2^24 x 1024): more than 2^32
     threads.  4096 rows repeated: every logit of the first and of the last
     4096."""
-    if torch.cuda.mem_get_info()[0] < 150 << 30:
-        pytest.skip("needs 120 GB of device memory")
+    if torch.cuda.mem_get_info()[0] < 110 << 30:
+        pytest.skip("needs 90 GB of device memory")
     T, H, E = 1 << 24, 400, 1024
     x = pkg.synth.activations(4096, H, 90, dev)
     W = _router(E, H, 91, dev)
