@@ -31,10 +31,10 @@
 // the current ones are used.
 //
 // Bound: the weights' bytes.  T = 96 over 256 experts (hidden 2048, inter
-// 512; about 245 experts active: 267 and 133 MB of weights): gate/up 62.6 us,
-// down 37.0 (4.3 and 3.6 TB/s, in a kernel trace; a bare read in the same
-// pattern reaches 6.1).  The call takes 108.5 us; with f16 (q - z) * s operands
-// in 512-thread blocks and three schedule launches it took 160.
+// 512; about 245 experts active: 267 and 133 MB of weights): gate/up 59.9 us,
+// down 35.7 (4.5 and 3.7 TB/s, in a kernel trace; a bare read in the same
+// pattern reaches 6.1).  The call takes 108 us; with f16 (q - z) * s operands in
+// 512-thread blocks and three schedule launches it took 160.
 #ifndef AIMA_GROUPED_THIN_H_
 #define AIMA_GROUPED_THIN_H_
 

@@ -806,7 +806,6 @@ static int check_routed_stack(const aima_moe_layer* layers, const aima_u4_tensor
   return AIMA_OK;
 }
 
-// The routed stack decode's launches on workspace w (its error word is w.err).
 namespace {
 
 // Layer input and router of the routed stack in one launch: logits = router .
@@ -854,6 +853,7 @@ static int norm_router_launch(const uint16_t* r, const aima_moe_layer& L, float 
 
 }  // namespace
 
+// The routed stack decode's launches on workspace w (its error word is w.err).
 static int routed_stack_run(const aima_moe_layer* layers, const aima_u4_tensor* routers,
                             int32_t n_layers, float eps, const uint16_t* residual_in, int32_t k,
                             float min_weight_sum, int32_t* ids, float* weights, uint16_t* out,

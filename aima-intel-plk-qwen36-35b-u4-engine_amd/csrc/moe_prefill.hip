@@ -978,8 +978,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(
 // write bandwidth while all blocks store).  Loading only the first group's
 // rows before multiplying measured 3 % slower, one barrier-ringed kernel of
 // 4 waves x 64 weight rows, two blocks per CU, 6 %.  T = 16384 (hidden 2048,
-// inter 512): 427 us a layer, grouped_gemm_kernel 490 (same box; MFMA-bound
-// 270 at the rate of a large f16 product).
+// inter 512): 427 us a layer, grouped_gemm_kernel 490 (one card, without a
+// trace; 397 to 423 in traces by card; MFMA-bound 270 at the rate of a large f16
+// product).
 constexpr int kDownRows = 128;
 constexpr int kDownGroups = 4;  // quantization groups along K
 constexpr int kDownTokens = kDownRows * kDownGroups * 256;  // bytes of LDS

@@ -65,8 +65,9 @@ class GroupedU4PrefillTiming:
     are already on the device); schedule_prepare_us: host work on the
     schedule's inputs before the run (moving host top-k rows and router
     weights to the device, repacking strided rows; 0 for dense device inputs
-    and for the native router); device_schedule_us: the device schedule
-    (count, scan, scatter kernels), median over the timed repeats from the
+    and for the native router); device_schedule_us: the device schedule (one
+    to three launches) and, for float32 hidden states, their rounding to f16,
+    which shares its first launch: median over the timed repeats from the
     stage events; schedule_upload_us equals it and schedule_setup_us is
     prepare + upload, as in the reference's device-schedule path
     (grouped_s8_u4_prefill_runtime.cpp:1165-1168).  The samples include the

@@ -393,8 +393,9 @@ typedef struct aima_prefill_options {
   int64_t topk_stride;    /* bytes between consecutive tokens' int32 top-k rows
                              (a multiple of 4, >= 4 * k); 0 = 4 * k (dense) */
   void* stage_events[5];  /* optional hipEvent_t, recorded on `stream` before the
-                             schedule and after the schedule, the gate/up GEMM,
-                             the down GEMM and the combine (NULL entries skipped) */
+                             schedule and after the schedule (which rounds an f32 x
+                             beside its first launch), the gate/up GEMM, the down
+                             GEMM and the combine (NULL entries skipped) */
   float* swiglu_f32;      /* optional f32 [rows][inter], 16-byte aligned: the SwiGLU
                              rows before their f16 rounding (RunLayer's
                              grouped_swiglu_f32); rows in schedule order, T*k routed
