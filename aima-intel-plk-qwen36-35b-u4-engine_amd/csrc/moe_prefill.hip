@@ -70,6 +70,9 @@ static int64_t tile_bound(const PrefillDims& d, int64_t bm) {
   return (d.A + bm - 1) / bm + std::min<int64_t>(d.E, d.A) + (d.T + bm - 1) / bm;
 }
 
+// Whether a turn's scales and zero points of a row are aligned for vector loads.
+static bool thin_aligned(const aima_u4_tensor& t) { return aligned(t.scale, 8) && aligned(t.zp, 2); }
+
 // Tile height.  16-row tiles in small blocks (several per CU:
 // grouped_thin_kernel) beat the 512-thread blocks of grouped_gemm_kernel while
 // most experts have few rows; but every 16 rows read an expert's weights
@@ -88,9 +91,11 @@ static int64_t tile_bound(const PrefillDims& d, int64_t bm) {
 //   T = 300 140 against 102; inter 1024, hidden 4096, k = 1, T = 1900 294
 //   against 182; uniform there: inter 768, T = 150 176 against 195, T = 300
 //   192 against 205.
-static int tile_rows_log2(const PrefillDims& d, bool with_shared) {
+// - scales and zero points off their vector alignment cost a 16-row tile more
+//   too: inter 512, k = 8, T = 300, Zipf 1.1 114 against 91 us, uniform 147 against 154.
+static int tile_rows_log2(const PrefillDims& d, bool with_shared, bool vectors) {
   const int64_t rows = d.A + (with_shared ? d.T : 0);
-  const int64_t most = d.I <= 512 ? 3200 : (13 << 16) / d.I;
+  const int64_t most = d.I <= 512 && vectors ? 3200 : (13 << 16) / std::max(d.I, 512);
   return d.A <= 10 * (int64_t)d.E && rows <= most ? kMinTileLog2 : 8;
 }
 
@@ -104,7 +109,11 @@ static PrefillDims prefill_dims(const aima_moe_layer* L, int64_t T, int k,
   d.H = L->hidden;
   d.I = L->inter;
   d.nb = (d.A + kSchedBlock - 1) / kSchedBlock;
-  d.bm_log2 = tile_rows_log2(d, with_shared);
+  const aima_u4_tensor* const w[] = {&L->gate_up, &L->up, &L->down, &L->shared_gate_up,
+                                     &L->shared_up, &L->shared_down};
+  bool vectors = true;
+  for (const aima_u4_tensor* t : w) vectors = vectors && thin_aligned(*t);
+  d.bm_log2 = tile_rows_log2(d, with_shared, vectors);
   d.max_tiles = tile_bound(d, 1 << d.bm_log2);
   return d;
 }
@@ -1467,7 +1476,7 @@ static int record(hipEvent_t e, hipStream_t st) {
 // whole turns along K, every row's run aligned.
 static bool thin_vectors(int64_t K, const aima_u4_tensor* const (&w)[4]) {
   bool ok = K % (128 * kThinTurn) == 0;
-  for (const aima_u4_tensor* t : w) ok = ok && aligned(t->scale, 8) && aligned(t->zp, 2);
+  for (const aima_u4_tensor* t : w) ok = ok && thin_aligned(*t);
   return ok;
 }
 

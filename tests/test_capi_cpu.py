@@ -367,21 +367,23 @@ def test_router_gemm_validation(pkg):
         assert L.size_query("aima_router_gemm_workspace_size", 8192, 2048, f32) == 0
 
 
-@pytest.mark.parametrize("H,I,E,k,shared,last", [
-    (2048, 512, 256, 8, False, 320),    # 10 assignments per expert
-    (2048, 512, 256, 8, True, 320),
-    (2048, 512, 256, 1, False, 2560),
-    (2048, 512, 256, 1, True, 1600),    # 3200 rows with the shared expert's
-    (2048, 512, 60, 1, True, 600),
-    (2048, 768, 256, 8, False, 138),    # 1109 rows
-    (2048, 768, 256, 8, True, 123),
-    (4096, 1024, 256, 1, True, 416),    # 832 rows
+@pytest.mark.parametrize("H,I,E,k,shared,off,last", [
+    (2048, 512, 256, 8, False, 0, 320),    # 10 assignments per expert
+    (2048, 512, 256, 8, True, 0, 320),
+    (2048, 512, 256, 1, False, 0, 2560),
+    (2048, 512, 256, 1, True, 0, 1600),    # 3200 rows with the shared expert's
+    (2048, 512, 60, 1, True, 0, 600),
+    (2048, 768, 256, 8, False, 0, 138),    # 1109 rows
+    (2048, 768, 256, 8, True, 0, 123),
+    (4096, 1024, 256, 1, True, 0, 416),    # 832 rows
+    (2048, 512, 256, 8, False, 2, 208),    # unaligned scales: 1664 rows
 ])
-def test_prefill_thin_tile_rule(pkg, H, I, E, k, shared, last):
+def test_prefill_thin_tile_rule(pkg, H, I, E, k, shared, off, last):
     """The most tokens of a call in 16-row tiles: beyond, skewed routing made
     them up to 1.7 times slower than 256-row ones."""
     L = pkg._lib
     lc = _fake_layer(pkg, H=H, I=I, E=E)
+    lc.down.scale += off
     rows, blocks, down = C.c_int32(), C.c_int32(), C.c_int32()
     for T, tile in ((1, 16), (last, 16), (last + 1, 256), (100000, 256)):
         L.call("aima_moe_prefill_tiling", C.byref(lc), T, k,
