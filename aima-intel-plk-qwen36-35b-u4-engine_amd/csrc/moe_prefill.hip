@@ -71,7 +71,9 @@ static int64_t tile_bound(const PrefillDims& d, int64_t bm) {
 }
 
 // Whether a turn's scales and zero points of a row are aligned for vector loads.
-static bool thin_aligned(const aima_u4_tensor& t) { return aligned(t.scale, 8) && aligned(t.zp, 2); }
+static bool thin_aligned(const aima_u4_tensor& t) {
+  return aligned(t.scale, 8) && aligned(t.zp, 2);
+}
 
 // Tile height.  16-row tiles in small blocks (several per CU:
 // grouped_thin_kernel) beat the 512-thread blocks of grouped_gemm_kernel while

@@ -330,17 +330,17 @@ def test_prefill_thin_tiles_unbiased(pkg, dev, H, I):
     assert abs(off) <= 6 * 2.0 ** -11 / np.sqrt(ref.size)
 
 
-@pytest.mark.parametrize("H,reps,more", [(2048, 4, 700), (2304, 4, 100)])
+@pytest.mark.parametrize("H,reps,more", [(2048, 4, 700), (2304, 4, 100), (768, 6, 1300)])
 @pytest.mark.parametrize("capture,shift", [(False, 0), (False, 1), (True, 0)])
 def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture, shift):
     """The down GEMM that keeps a tile's token rows in LDS (inter 512, over 32
     assignments per expert, at least 384 blocks at hidden 1536 and more):
     remainders around each 32-row block of both 128-row halves, thin halves, and
-    a column count that leaves waves of a block without a chunk (2304).  Scales
-    and zero points off their vector alignment (shift) take the instance that
-    loads them value by value.  With the f32 copies requested, the f16
-    contributions are those values rounded.  Tolerance as the other prefill
-    tests."""
+    a column count that leaves waves of a block without a chunk (2304); the same
+    at hidden 768, where the rows are not kept.  Scales and zero points off
+    their vector alignment (shift) take the instance that loads them value by
+    value.  With the f32 copies requested, the f16 contributions are those values
+    rounded.  Tolerance as the other prefill tests."""
     I = 512
     counts = [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 256, 289] * reps + [more]
     layer = pkg.synth.moe_layer(hidden=H, inter=I, experts=len(counts), seed=400 + H, device=dev)
@@ -348,7 +348,8 @@ def test_prefill_resident_down_rows(pkg, dev, H, reps, more, capture, shift):
     ids = np.repeat(np.arange(len(counts)), counts).astype(np.int32)
     ids = np.random.default_rng(H + I).permutation(ids)[:, None].copy()
     T = len(ids)
-    assert T > 32 * len(counts) and -(-2 * T // 128) * -(-H // 512) >= 384
+    assert T > 32 * len(counts) and -(-2 * T // 128) * -(-H // 512) >= 320
+    assert pkg.prefill_tiling(layer, T, 1)[2] == (128 if H >= 1536 else 256)
     if shift:
         _off_alignment(layer)
     x = pkg.synth.activations(T, H, 401, dev)
